@@ -1,0 +1,89 @@
+"""GPU parity of the small-output GEMM kernels at the edges of their tiles and of the rules that choose them.
+
+wf_gemm_bf16: the few-row kernel (1-16 rows; to 64 with SiLU on the input), the LDS tiles of gemm_small.hpp (32 x 64
+and 64 x 64 with K split over groups of waves, 64 x 128, 128 x 128) and the direct kernel behind them; sizes one
+off a tile, K tails inside a 64-element step, rows and columns past the end, strided A and y, a bias that is only
+2-byte aligned, no bias.
+
+Bound per element, against the product in 64 bits: fp32 accumulation in any order, K 2^-23 sum |a w| (with
+margin 2 over (K - 1) 2^-24), then one bf16 rounding (half an ulp of 8 significand bits: 2^-8 of the value); an
+activation has slope at most 1.13 and adds a rounding of its own and the hardware exponential's and reciprocal's few ulps (2^-20).
+"""
+
+import pytest
+import torch
+
+from waveforcing_amd import _lib
+from waveforcing_amd.dit import gemm_bf16
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _rand(shape, seed, std=1.0):
+    return (torch.randn(shape, generator=torch.Generator().manual_seed(seed)) * std).to(torch.bfloat16).to(DEV)
+
+
+def _check_bf16(got, a, w, b, silu_in, act):
+    a64, w64 = a.double(), w.double()
+    if silu_in:  # rounded to bf16 as the module's output; the kernel's own rounding may differ by an ulp
+        slack = (a64 * torch.sigmoid(a64)).abs() * 2.0 ** -8
+        a64 = a64 * torch.sigmoid(a64)
+    else:
+        slack = torch.zeros_like(a64)
+    pre = a64 @ w64.t() + (0 if b is None else b.double())
+    err = a.shape[1] * 2.0 ** -23 * (a64.abs() @ w64.abs().t()) + slack @ w64.abs().t() + 2.0 ** -8 * pre.abs()
+    ref = pre
+    if act == "silu":
+        ref = pre * torch.sigmoid(pre)
+    elif act == "gelu":
+        ref = torch.nn.functional.gelu(pre, approximate="tanh")
+    bound = (1.13 * err + (2.0 ** -8 + 2.0 ** -20) * ref.abs() if act else err) * 1.01 + 1e-30
+    worst = ((got.double() - ref).abs() / bound).max().item()
+    assert worst <= 1.0, f"{worst:.3f} of the bound"
+
+
+@pytest.mark.parametrize("M,K,N,silu_in,act", [
+    (1, 8, 4, False, None), (1, 256, 1536, False, "silu"), (3, 1536, 9216, True, None), (8, 72, 20, True, "gelu"),
+    (9, 1544, 60, False, "gelu"), (16, 520, 17 * 4, True, "silu"), (16, 1536, 16, False, None),
+    (17, 64, 64, True, None), (33, 200, 36, True, "silu"), (64, 136, 132, True, None), (65, 264, 68, True, "gelu"),
+    (17, 72, 60, False, None), (32, 512, 64, False, "gelu"), (33, 1032, 68, False, "silu"), (300, 4096, 1536, False, "gelu"),
+    (512, 4096, 1536, False, "gelu"), (513, 1544, 1540, False, None), (780, 1536, 1536, False, None),
+    (1100, 520, 2052, False, None), (4680, 64, 1536, False, None), (129, 192, 4100, False, "silu"),
+    (2000, 328, 2500, False, None), (4680, 1536, 64, False, None),
+])
+def test_gemm_bf16_tiles(M, K, N, silu_in, act):
+    a, w, b = _rand((M, K), M + K), _rand((N, K), N, 0.05), _rand((N,), 7)
+    _check_bf16(gemm_bf16(a, w, b, silu_in=silu_in, act_out=act), a, w, b, silu_in, act)
+
+
+@pytest.mark.parametrize("M,K,N", [(3, 264, 20), (40, 264, 36), (300, 264, 500), (700, 1032, 3000)])
+def test_gemm_bf16_strides_bias_and_edges(M, K, N):
+    """A with a row stride, y with an odd multiple of 4, a bias 2 bytes off, no bias; nothing past y's columns or
+    rows is written."""
+    big = _rand((M, K + 40), 11)
+    a, w = big[:, :K], _rand((N, K), 12, 0.05)
+    bias = _rand((N + 1,), 13)[1:]
+    assert bias.data_ptr() % 4 == 2
+    for b in (bias, None):
+        y = torch.full((M + 2, N + 12), 3.0, dtype=torch.bfloat16, device=DEV)
+        gemm_bf16(a, w, b, out=y[:M, :N])
+        _check_bf16(y[:M, :N], a, w, b, False, None)
+        assert bool((y[M:] == 3.0).all()) and bool((y[:, N:] == 3.0).all())
+
+
+def test_gemm_bf16_zero_without_bias_keeps_its_sign():
+    """A product of -0 without a bias stays -0 (the tiles add a bias of -0, never +0)."""
+    a = torch.zeros((40, 64), dtype=torch.bfloat16, device=DEV)
+    w = -torch.ones((64, 64), dtype=torch.bfloat16, device=DEV)
+    assert torch.equal(gemm_bf16(a, w, None), a.float().matmul(w.float().t()).to(torch.bfloat16))
+
+
+def test_flags_and_shapes_still_refused():
+    a, w = _rand((4, 64), 1), _rand((8, 64), 2)
+    y = torch.empty((4, 8), dtype=torch.bfloat16, device=DEV)
+    st = _lib.stream_handle(torch.device(DEV))
+    for args in ((4, 60, 64, 8, 8, 0), (4, 64, 64, 6, 8, 0), (4, 64, 64, 8, 8, 8), (4, 64, 64, 8, 8, 6), (4, 64, 60, 8, 8, 0)):
+        m, k, lda, n, ldy, flags = args
+        with pytest.raises(RuntimeError):
+            _lib.call("wf_gemm_bf16", a.data_ptr(), m, k, lda, w.data_ptr(), n, None, y.data_ptr(), ldy, flags, st)

@@ -18,33 +18,162 @@
 //    layout the wavefront hands on (backend.py:456-490), converted to bf16
 //    as torch converts float64 (through float32).
 //
-// GEMM structure: a workgroup of 4 waves owns a 64 x 128 output tile, each
-// wave 32 rows x 64 columns as two v_mfma_f32_32x32x16_bf16 blocks.  The
-// operand fragments of that MFMA are 16 contiguous bytes of one row of A
-// and of W (lane l: row l % 32, K elements 8 (l / 32) .. + 7), so they are
-// loaded straight from global memory (neighbouring K steps share cache
-// lines), one K step ahead of the MFMAs.  Each wave's results go out through
-// its own LDS rows as 128-byte row segments.  These GEMMs are a few percent
-// of a chunk's work (0.9 GFLOP for the patch embedding or the head at 1.3B).
+// The GEMM has three forms, chosen by size in wf_gemm_bf16: few rows (the W stream bounds it), LDS tiles
+// (gemm_small.hpp) and the direct kernel for what the other two do not take.
 #include <type_traits>
 
+#include "gemm_core.hpp"
+#include "gemm_small.hpp"
 #include "wf_common.hpp"
 
 namespace wf {
 namespace {
 
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef float v16f __attribute__((ext_vector_type(16)));
+using namespace gemm;
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+__device__ inline float bf16_round(float x) { return __uint_as_float(pack_bf16x2_hw(x, 0.f) << 16); }
+
+struct Bf16GemmArgs {
+  const uint16_t* a;
+  const uint16_t* w;
+  const uint16_t* bias;
+  uint16_t* y;
+  int64_t lda, ldy;
+  int M, N, K;
+  int act;      // 0 none, 1 SiLU, 2 GELU(tanh)
+  int m_tiles;  // groups of kSkinnyRows rows
+};
 
 constexpr int kWaves = 4;
 constexpr int kTileM = 64, kTileN = 128;
 
-// x * sigmoid(x) = x / (1 + e^-x), on the hardware exponential and reciprocal.
-__device__ inline float silu(float x) {
-  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x));
-}
+constexpr int kSkinnyRows = 16;   // rows of A per workgroup
+constexpr int kSkinnyCols = 16;   // columns of y (rows of W) per workgroup
+constexpr int kSkinnyWaves = 4;   // waves per workgroup, which split K
+constexpr int kSkinnyRing = 4;    // pieces of 64 K elements a wave has in flight
+constexpr int kPieceBytes = kSkinnyCols * 128;
 
-__device__ inline float bf16_round(float x) { return __uint_as_float(pack_bf16x2_hw(x, 0.f) << 16); }
+// y for up to 16 rows of A (8 with NA = 1) and 16 rows of W, the few-row products of the time embedding.  The
+// bound is the stream of W: K goes to the four waves in pieces of 64 elements (whole 128-byte lines of every W
+// row), which each wave brings into its own LDS ring by DMA, four pieces ahead, without a barrier.  A piece of A
+// is loaded, SiLU'd and handed over in LDS by the wave itself, 16 bytes per lane, so that the activation costs
+// what the rows hold and not a 16-row tile.  v_mfma_f32_16x16x32_bf16 takes 16 bytes of one row per lane (row
+// l % 16, K elements 8 (l / 16) .. + 7); chunk c of row r lies at 16 (c ^ ((r / 2) % 8)).  The waves' partial
+// sums are added in wave order.
+template <bool SILU_IN, int NA>
+__global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_bf16_skinny_kernel(Bf16GemmArgs p) {
+  constexpr int P = kSkinnyRing;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kSkinnyWaves * (P * kPieceBytes + kSkinnyRows * 128)];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, kq = lane >> 4;
+  const int m0 = static_cast<int>(blockIdx.x % static_cast<uint32_t>(p.m_tiles)) * kSkinnyRows;
+  const int n0 = static_cast<int>(blockIdx.x / static_cast<uint32_t>(p.m_tiles)) * kSkinnyCols;
+  const int rows = min(p.M - m0, kSkinnyRows), cols = min(p.N - n0, kSkinnyCols);
+  uint8_t* const ring = lds + wave * (P * kPieceBytes);
+  uint8_t* const aw = lds + kSkinnyWaves * P * kPieceBytes + wave * (kSkinnyRows * 128);
+  // rows past M / N and chunks past K read zeros
+  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(p.a + static_cast<int64_t>(m0) * p.lda), 0,
+      ((rows - 1) * static_cast<int>(p.lda) + p.K) * 2, kBufferRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(p.w + static_cast<int64_t>(n0) * p.K), 0, cols * p.K * 2, kBufferRsrcWord3);
+  // Lane l moves chunk l % 8 of row l / 8 (+ 8 i) of A, and of W the chunk that belongs at position l % 8 there.
+  const int r8 = lane >> 3, c8 = lane & 7;
+  u32x4 ar[P][NA];
+  int aoff[NA], woff[2], wk[2];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) aoff[i] = ((r8 + 8 * i) * static_cast<int>(p.lda) + 8 * c8) * 2;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    wk[i] = 8 * (c8 ^ (((r8 + 8 * i) >> 1) & 7));
+    woff[i] = ((r8 + 8 * i) * p.K + wk[i]) * 2;
+  }
+  auto load = [&](auto S, int piece) {
+    constexpr int s = decltype(S)::value;
+    const int k0 = 64 * (wave + kSkinnyWaves * piece);
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+      ar[s][i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, k0 + 8 * c8 < p.K ? aoff[i] + 2 * k0 : kOutOfRange, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      dma16(rsrc_w, ring + s * kPieceBytes + i * 1024, k0 + wk[i] < p.K ? woff[i] + 2 * k0 : kOutOfRange);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  v4f acc = {0, 0, 0, 0};
+  const int x = (r16 >> 1) & 7;
+  auto compute = [&](auto S) {
+    constexpr int s = decltype(S)::value;
+    // this piece's loads landed; those of the P - 1 pieces behind it may be in flight
+    wait_counts<(P - 1) * (2 + NA), 15>();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      u32x4 v = ar[s][i];
+      if constexpr (SILU_IN) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = pack_bf16x2_hw(silu(bf16_lo_to_f32(v[e])), silu(bf16_hi_to_f32(v[e])));
+      }
+      const int r = r8 + 8 * i;
+      *reinterpret_cast<u32x4*>(aw + r * 128 + 16 * (c8 ^ ((r >> 1) & 7))) = v;
+    }
+    // read back by other lanes of this wave: LDS executes a wave's accesses in order (with NA = 1 rows 8.. hold
+    // whatever is there; they only reach rows of y that are not stored)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    v8bf av[2], wv[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int at = r16 * 128 + 16 * ((4 * u + kq) ^ x);
+      wv[u] = *reinterpret_cast<const v8bf*>(ring + s * kPieceBytes + at);
+      av[u] = *reinterpret_cast<const v8bf*>(aw + at);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[u], av[u], acc, 0, 0, 0);
+    // the piece's fragments are in registers before its slot is filled again
+    wait_counts<63, 0>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  const int pieces = ((p.K + 63) / 64 + kSkinnyWaves - 1) / kSkinnyWaves;  // the last ones of a wave may be past K
+  static_for<P>([&](auto S) { load(S, decltype(S)::value); });
+  for (int i = 0; i < pieces; i += P) {
+    static_for<P>([&](auto S) {
+      constexpr int s = decltype(S)::value;
+      compute(S);                 // past the end: zeros
+      load(S, i + s + P);
+    });
+  }
+  wait_counts<0, 0>();
+  __syncthreads();
+  v4f* const red = reinterpret_cast<v4f*>(lds);
+  red[wave * 64 + lane] = acc;
+  __syncthreads();
+  if (wave > 0) return;
+  // the lane's row m0 + l % 16, columns n0 + 4 (l / 16) .. + 3
+  v4f t = acc;
+#pragma unroll
+  for (int s = 1; s < kSkinnyWaves; ++s) {
+    const v4f o = red[s * 64 + lane];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t[e] = t[e] + o[e];
+  }
+  const int m = m0 + r16, n = n0 + 4 * kq;
+  if (m >= p.M || n >= p.N) return;
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] = bf16_round(p.bias ? __fadd_rn(t[e], bf16_bits_to_f32(p.bias[n + e])) : t[e]);
+    if (p.act == 1) v[e] = silu(v[e]);
+    if (p.act == 2) v[e] = gelu_tanh(v[e]);
+  }
+  *reinterpret_cast<uint2*>(p.y + static_cast<int64_t>(m) * p.ldy + n) =
+      make_uint2(pack_bf16x2_hw(v[0], v[1]), pack_bf16x2_hw(v[2], v[3]));
+}
 
 template <bool SILU_IN>
 __device__ inline v8bf load_frag(const uint16_t* row, int k, int K) {
@@ -61,17 +190,11 @@ __device__ inline v8bf load_frag(const uint16_t* row, int k, int K) {
   return __builtin_bit_cast(v8bf, v);
 }
 
-struct Bf16GemmArgs {
-  const uint16_t* a;
-  const uint16_t* w;
-  const uint16_t* bias;
-  uint16_t* y;
-  int64_t lda, ldy;
-  int M, N, K;
-};
-
-// ACT_OUT: 0 none, 1 SiLU, 2 GELU(tanh).
-template <bool SILU_IN, int ACT_OUT>
+// The general form: any size, 64-bit row addresses.  A workgroup of 4 waves owns a 64 x 128 output tile, each wave
+// 32 rows x 64 columns as two v_mfma_f32_32x32x16_bf16 blocks whose fragments (16 contiguous bytes of one row of
+// A and of W: lane l row l % 32, K elements 8 (l / 32) .. + 7) come straight from global memory, one K step
+// ahead of the MFMAs.  A latency chain per K step; it serves what the kernels above do not take.
+template <bool SILU_IN>
 __global__ __launch_bounds__(kWaves * 64) void gemm_bf16_kernel(Bf16GemmArgs p) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -116,8 +239,8 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_bf16_kernel(Bf16GemmArgs p) 
         float t = acc[4 * g + e];
         if (p.bias && n < p.N) t = __fadd_rn(t, bf16_bits_to_f32(p.bias[n + e]));
         t = bf16_round(t);
-        if constexpr (ACT_OUT == 1) t = silu(t);
-        if constexpr (ACT_OUT == 2) t = gelu_tanh(t);
+        if (p.act == 1) t = silu(t);
+        if (p.act == 2) t = gelu_tanh(t);
         v[e] = t;
       }
       *reinterpret_cast<uint2*>(yw + l32 * YP + 2 * (32 * j + 8 * g + 4 * half)) =
@@ -188,10 +311,17 @@ __global__ __launch_bounds__(256) void unpatchify_x0_kernel(const uint16_t* __re
   *reinterpret_cast<uint32_t*>(out + (((b * F + f) * C + c) * H + yy) * static_cast<int64_t>(W) + 2 * xp) = o;
 }
 
-template <bool SILU_IN, int ACT>
-void launch_gemm(const Bf16GemmArgs& p, hipStream_t st) {
+template <bool SILU_IN, int NA>
+void launch_skinny(const Bf16GemmArgs& p, hipStream_t st) {
+  const int64_t blocks = static_cast<int64_t>(p.m_tiles) * ((p.N + kSkinnyCols - 1) / kSkinnyCols);
+  hipLaunchKernelGGL((gemm_bf16_skinny_kernel<SILU_IN, NA>), dim3(static_cast<uint32_t>(blocks)),
+                     dim3(kSkinnyWaves * 64), 0, st, p);
+}
+
+template <bool SILU_IN>
+void launch_direct(const Bf16GemmArgs& p, hipStream_t st) {
   const dim3 grid((p.N + kTileN - 1) / kTileN, (p.M + kTileM - 1) / kTileM);
-  hipLaunchKernelGGL((gemm_bf16_kernel<SILU_IN, ACT>), grid, dim3(kWaves * 64), 0, st, p);
+  hipLaunchKernelGGL(gemm_bf16_kernel<SILU_IN>, grid, dim3(kWaves * 64), 0, st, p);
 }
 
 bool a16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -219,27 +349,41 @@ int wf_gemm_bf16(const void* a, int64_t m, int64_t k, int64_t lda, const void* w
   WF_REQUIRE((flags & ~(WF_BF16_SILU_IN | WF_BF16_SILU_OUT | WF_BF16_GELU_OUT)) == 0 &&
                  !((flags & WF_BF16_SILU_OUT) && (flags & WF_BF16_GELU_OUT)),
              WF_E_INVALID, "%s: bad flags 0x%x", fn, flags);
-  wf::Bf16GemmArgs p;
-  p.a = static_cast<const uint16_t*>(a);
-  p.w = static_cast<const uint16_t*>(w);
-  p.bias = static_cast<const uint16_t*>(bias);
-  p.y = static_cast<uint16_t*>(y);
-  p.lda = lda;
-  p.ldy = ldy;
-  p.M = static_cast<int>(m);
-  p.N = static_cast<int>(n);
-  p.K = static_cast<int>(k);
   hipStream_t st = wf::as_stream(stream);
   const bool silu_in = (flags & WF_BF16_SILU_IN) != 0;
-  if (silu_in) {
-    if (act == 0) wf::launch_gemm<true, 0>(p, st);
-    else if (act == 1) wf::launch_gemm<true, 1>(p, st);
-    else wf::launch_gemm<true, 2>(p, st);
-  } else {
-    if (act == 0) wf::launch_gemm<false, 0>(p, st);
-    else if (act == 1) wf::launch_gemm<false, 1>(p, st);
-    else wf::launch_gemm<false, 2>(p, st);
+  constexpr int64_t kSpan = (1ll << 31) - 16;  // buffer offsets are 32-bit
+  wf::Bf16GemmArgs p{static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(w),
+                     static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(y), lda, ldy,
+                     static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), act, 0};
+  // Few rows (the time embedding's 1-21 frames): the W stream's kernel; 3 x 1536 -> 9216 with SiLU 9.4 us against
+  // 40.7 us for the direct kernel (28.3 MB of W), 3 x 5120 -> 30720 57 us (5.5 TB/s).  It takes 16 rows at a time
+  // and W again for each 16, so without SiLU the tiles take over at 17 rows (21 x 1536 -> 1536: 5.9 against
+  // 7.8 us); with it, which only this kernel and the direct one apply, at 65.
+  const int64_t skinny_max = silu_in ? 64 : wf::kSkinnyRows;
+  if (m <= skinny_max && wf::product_below({wf::kSkinnyRows, lda, 2}, kSpan) &&
+      wf::product_below({wf::kSkinnyCols, k, 2}, kSpan)) {
+    p.m_tiles = static_cast<int>((m + wf::kSkinnyRows - 1) / wf::kSkinnyRows);
+    if (silu_in)
+      m <= 8 ? wf::launch_skinny<true, 1>(p, st) : wf::launch_skinny<true, 2>(p, st);
+    else
+      m <= 8 ? wf::launch_skinny<false, 1>(p, st) : wf::launch_skinny<false, 2>(p, st);
+    return wf::check_launch(fn);
   }
+  // LDS-tiled: 512 x 4096 -> 1536 with GELU 15.0 us against 97.8 us, 4680 x 1536 -> 64 (head) 7.5 against 28.6 us,
+  // 4680 x 64 -> 1536 (patch embedding) 8.4 against 13.2 us for the direct kernel.
+  if (!silu_in && wf::product_below({m + 256, lda, 2}, kSpan) && wf::product_below({n + 256, k, 2}, kSpan)) {
+    const wf::gemm::SmallArgs q{a, w, nullptr, nullptr, p.bias, p.y, p.M, p.N, 2 * p.K, static_cast<int>(2 * lda), ldy,
+                                ldy % 8 == 0 && wf::a16(y), (reinterpret_cast<uintptr_t>(bias) & 7u) == 0};
+    const int tile = wf::gemm::pick_small(p.M, p.N, q.kb, true);
+    if (act == 0)
+      wf::gemm::launch_small<wf::gemm::OpBf16, 0>(tile, q, st);
+    else if (act == 1)
+      wf::gemm::launch_small<wf::gemm::OpBf16, 1>(tile, q, st);
+    else
+      wf::gemm::launch_small<wf::gemm::OpBf16, 2>(tile, q, st);
+    return wf::check_launch(fn);
+  }
+  silu_in ? wf::launch_direct<true>(p, st) : wf::launch_direct<false>(p, st);
   return wf::check_launch(fn);
 }
 

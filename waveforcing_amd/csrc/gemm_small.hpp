@@ -1,0 +1,376 @@
+// GEMM for outputs that do not fill the GPU with the 128 x 256 / 256 x 256 tiles of gemm_w8a8.hip, and for the
+// bf16 linears: y[m,n] = epilogue(sum_k a[m,k] * w[n,k]), int8, e4m3 or bf16 operands.
+//
+// What bounds it: with few tiles neither the matrix cores nor memory, but the time of one K step in a workgroup
+// (barrier, fragment reads, a chain of MFMAs) times the steps, and below that the operand stream, (BM + BN) rows
+// of K through the 64 B/clk vector-memory path of one CU.  So the tiles are small (more CUs share the stream), the
+// smallest split K over groups of waves, fragments are read a step ahead of their MFMAs, and the LDS ring keeps up
+// to ST - 1 steps in flight.  Bytes move global -> LDS by DMA in the layout of gemm_w8a8.hip (1 KB blocks of 8 rows,
+// K chunks swizzled by the row), and without a K split every output sees the same MFMAs in the same K order as
+// there: bit-identical results (int32 sums with a split, too).
+//
+// One K step: wait for the own DMAs of step kb, barrier (every wave's have landed and every wave is done with
+// step kb - 1's stage), read step kb's fragments, DMA step kb + ST - 1 into that freed stage, then the MFMAs of
+// step kb - 1.  DMAs past K read zeros into stages that nobody reads any more.
+#pragma once
+
+#include <type_traits>
+
+#include "gemm_core.hpp"
+
+namespace wf {
+namespace gemm {
+
+// BM x BN outputs per workgroup of KS groups of WM x WN waves, each wave (BM / WM) x (BN / WN) in 32 x 32 blocks;
+// group g takes K steps g, g + KS, ... through its own ring of ST LDS stages, and the groups' sums are added at
+// the end (KS > 1 changes the order of fp32 sums, never an int32 one).
+template <int BM_, int BN_, int WM_, int WN_, int ST_, int KS_ = 1>
+struct SmallTile {
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, ST = ST_, KS = KS_;
+  static constexpr int NW = WM * WN, THREADS = KS * NW * 64;  // NW: waves of one group
+  static constexpr int MI = BM / WM / 32, NI = BN / WN / 32;
+  static constexpr int NBA = BM / 8 / NW, NBB = BN / 8 / NW, NDMA = NBA + NBB;
+  static constexpr int STAGE = (BM + BN) * BK;
+  static constexpr int WPITCH = BN / WN * 2 + 16;   // row pitch of a wave's 32-row output slab
+  static constexpr int SLABS = MI > 1 ? 2 : 1;
+  static_assert(MI >= 1 && NI >= 1 && MI * WM * 32 == BM && NI * WN * 32 == BN, "32 x 32 blocks");
+  static_assert(NBA * 8 * NW == BM && NBB * 8 * NW == BN, "DMA blocks");
+  static_assert(ST >= 3 && NDMA * (ST - 2) < 64, "outstanding DMAs");
+  static constexpr int LDS = KS * ST * STAGE;
+  static constexpr int ACC = MI * NI * 64 * 64;     // one wave's sums (bytes)
+  static_assert(NW * SLABS * 32 * WPITCH <= LDS && LDS <= 160 * 1024, "LDS of one workgroup");
+  static_assert(KS == 1 || (KS - 1) * NW * ACC <= LDS, "the groups' sums fit the stages");
+};
+
+struct SmallArgs {
+  const void* a;         // [M] rows of kb bytes, lda bytes apart
+  const void* w;         // [N] rows of kb bytes
+  const float* sx;       // int8: [M];  e4m3: [1]
+  const float* sw;       // int8: [N];  e4m3: [1]
+  const uint16_t* bias;  // [N] bf16 or null
+  uint16_t* y;           // [M, N] bf16 (ldy)
+  int M, N, kb, lda;
+  int64_t ldy;
+  int vec16;             // y and ldy allow 16-byte row stores
+  int bias8;             // bias is 8-byte aligned
+};
+
+// ACT, on the bf16 result: 0 none, 1 SiLU, 2 GELU(tanh).
+template <typename T, typename OP, int ACT>
+__global__ __launch_bounds__(T::THREADS) void gemm_small_kernel(SmallArgs p) {
+  constexpr int BM = T::BM, BN = T::BN, WN = T::WN, NW = T::NW, MI = T::MI, NI = T::NI, ST = T::ST;
+  constexpr int STAGE = T::STAGE, NBA = T::NBA, NDMA = T::NDMA, WPITCH = T::WPITCH;
+  constexpr bool kI8 = std::is_same<OP, OpI8>::value, kFp8 = std::is_same<OP, OpFp8>::value;
+  constexpr int SUB = OP::SUB, PIECES = OP::PIECES;
+  constexpr int CPS = BK / 16 / SUB;
+  constexpr int KS = T::KS;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds_all[T::LDS];
+
+  // Tiles in bands of GROUP_M tile rows swept column by column, a contiguous range of them per XCD.
+  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
+  const int n_tiles = tiles_m * tiles_n;
+  const int per_xcd = (n_tiles + NUM_XCD - 1) / NUM_XCD;
+  const int t = (blockIdx.x % NUM_XCD) * per_xcd + blockIdx.x / NUM_XCD;
+  if (blockIdx.x / NUM_XCD >= per_xcd || t >= n_tiles) return;
+  const int per_group = GROUP_M * tiles_n;
+  const int first_m = (t / per_group) * GROUP_M;
+  const int band = min(tiles_m - first_m, GROUP_M);
+  const int m0 = (first_m + (t % per_group) % band) * BM;
+  const int n0 = ((t % per_group) / band) * BN;
+
+  const int lane = threadIdx.x & 63;
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = KS > 1 ? wave_all % NW : wave_all, ks = KS > 1 ? wave_all / NW : 0;
+  uint8_t* const lds = lds_all + ks * (ST * STAGE);
+  const int wm = wave / WN, wn = wave % WN;
+  const int l32 = lane & 31, half = lane >> 5;
+
+  const __amdgpu_buffer_rsrc_t rsrc_a =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.a), 0, (p.M - 1) * p.lda + p.kb, kBufferRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rsrc_w =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.w), 0, p.N * p.kb, kBufferRsrcWord3);
+
+  // DMA block j of this wave: rows (j * NW + wave) * 8 .. + 7 of A (j < NBA) or of W.
+  int doff[NDMA], dcol[NDMA];
+#pragma unroll
+  for (int j = 0; j < NDMA; ++j) {
+    const bool is_a = j < NBA;
+    const int r = ((is_a ? j : j - NBA) * NW + wave) * 8 + (lane >> 3);
+    const int c = (lane & 7) ^ ((r >> 1) & 7);
+    dcol[j] = c * 16;
+    doff[j] = is_a ? (m0 + r) * p.lda + c * 16 : (n0 + r) * p.kb + c * 16;
+  }
+  // The group's step kb (step KS kb + ks of the whole) into stage STG.
+  auto dma_step = [&](int kb, auto STG) {
+    constexpr int stage = decltype(STG)::value;
+    const int k0 = (KS * kb + ks) * BK;
+    auto issue = [&](auto WHOLE) {
+      static_for<NDMA>([&](auto J) {
+        constexpr int j = decltype(J)::value;
+        uint8_t* const dst = lds + stage * STAGE + (j < NBA ? j * NW : BM / 8 + (j - NBA) * NW) * 1024 + wave * 1024;
+        const int off = decltype(WHOLE)::value || dcol[j] < p.kb - k0 ? doff[j] + k0 : kOutOfRange;
+        dma16(j < NBA ? rsrc_a : rsrc_w, dst, off);
+      });
+    };
+    // a whole step within K needs no check per chunk (rows past M and N are past the buffers' ends)
+    if (k0 + BK <= p.kb)
+      issue(ic<1>{});
+    else
+      issue(ic<0>{});
+  };
+
+  // Epilogue operands of the lane's outputs (block (j, i): row m = l32, columns 8 g + 4 half + 0..3 of block j),
+  // loaded ahead of the operand stream.  N % 4 == 0: a group of 4 columns is inside N or not at all.
+  float sxv[MI];
+  float scale = 1.f;
+  float4 swv[NI][4];
+  uint2 bv[NI][4];
+  if constexpr (kI8) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) sxv[i] = p.sx[min(m0 + (wm * MI + i) * 32 + l32, p.M - 1)];
+  }
+  if constexpr (kFp8) scale = p.sx[0] * p.sw[0];
+  auto col = [&](int j, int g) { return min(n0 + (wn * NI + j) * 32 + 8 * g + 4 * half, p.N - 4); };
+#pragma unroll
+  for (int j = 0; j < NI; ++j)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      bv[j][g] = make_uint2(0x80008000u, 0x80008000u);  // no bias: -0, which leaves every sum as it is
+      if constexpr (kI8) swv[j][g] = *reinterpret_cast<const float4*>(p.sw + col(j, g));
+    }
+  if (p.bias != nullptr) {
+    if (p.bias8) {
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) bv[j][g] = *reinterpret_cast<const uint2*>(p.bias + col(j, g));
+    } else {
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const uint16_t* b = p.bias + col(j, g);
+          bv[j][g] = make_uint2(b[0] | (static_cast<uint32_t>(b[1]) << 16), b[2] | (static_cast<uint32_t>(b[3]) << 16));
+        }
+    }
+  }
+
+  // Fragment pieces: sub-step s, lane half h, piece e is K chunk c = s*CPS + h*PIECES + e of the lane's row R,
+  // at R*128 + 16*(c ^ ((R/2)%8)).
+  const int x = (l32 >> 1) & 7;
+  const int lane_a = (wm * MI * 32 + l32) * BK;
+  const int lane_b = BM * BK + (wn * NI * 32 + l32) * BK;
+  int koff[SUB][PIECES];
+#pragma unroll
+  for (int s = 0; s < SUB; ++s)
+#pragma unroll
+    for (int e = 0; e < PIECES; ++e) koff[s][e] = 16 * ((s * CPS + half * PIECES + e) ^ x);
+
+  typename OP::acc_t acc[NI][MI];
+#pragma unroll
+  for (int j = 0; j < NI; ++j)
+#pragma unroll
+    for (int i = 0; i < MI; ++i) acc[j][i] = typename OP::acc_t{};
+
+  const int nk = ((p.kb + BK - 1) / BK + KS - 1) / KS;  // steps per group (a last one past K adds zeros)
+  static_for<ST - 1>([&](auto S) { dma_step(decltype(S)::value, S); });
+  // Fragments in two register sets: step kb's are read while the MFMAs of step kb - 1 run.  The stages and the
+  // sets are compile-time (the loop is unrolled over both), so a step costs no address arithmetic but its DMAs'.
+  v4i fa[2][SUB][MI][PIECES], fw[2][SUB][NI][PIECES];
+  auto mma = [&](auto B) {
+    constexpr int b = decltype(B)::value;
+#pragma unroll
+    for (int s = 0; s < SUB; ++s)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int i = 0; i < MI; ++i) acc[j][i] = OP::mfma(fw[b][s][j], fa[b][s][i], acc[j][i]);
+  };
+  auto fetch = [&](auto B, auto STG, int kb) {
+    constexpr int b = decltype(B)::value, stage = decltype(STG)::value;
+    // own DMAs of step kb landed (those of the ST - 2 steps behind it may be in flight), own reads of the stage
+    // before it done; the barrier makes both hold for every wave
+    wait_counts<NDMA * (ST - 2), 0>();
+    if constexpr (KS * NW > 1) __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const uint8_t* st = lds + stage * STAGE;
+#pragma unroll
+    for (int s = 0; s < SUB; ++s)
+#pragma unroll
+      for (int e = 0; e < PIECES; ++e) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+          fa[b][s][i][e] = *reinterpret_cast<const v4i*>(st + i * 32 * BK + (lane_a + koff[s][e]));
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+          fw[b][s][j][e] = *reinterpret_cast<const v4i*>(st + j * 32 * BK + (lane_b + koff[s][e]));
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    dma_step(kb + ST - 1, ic<(stage + ST - 1) % ST>{});
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  fetch(ic<0>{}, ic<0>{}, 0);
+  constexpr int UNROLL = ST % 2 == 0 ? ST : 2 * ST;
+  for (int kb = 1; kb < nk;) {
+    static_for<UNROLL>([&](auto U) {
+      constexpr int u = decltype(U)::value + 1;
+      if (kb < nk) {
+        fetch(ic<u & 1>{}, ic<u % ST>{}, kb);
+        mma(ic<(u & 1) ^ 1>{});
+        ++kb;
+      }
+    });
+  }
+  if (nk & 1)
+    mma(ic<0>{});
+  else
+    mma(ic<1>{});
+  // every DMA landed and every wave past its last LDS read before the stages are reused for the output staging
+  wait_counts<0, 0>();
+  if constexpr (KS * NW > 1) __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+
+  if constexpr (KS > 1) {
+    // groups 1.. hand their sums to group 0 (16 bytes per lane and store), which adds them in group order and
+    // finishes alone
+    typedef typename std::conditional<kI8, int, float>::type elem;
+    typedef elem v4e __attribute__((ext_vector_type(4)));
+    v4e* const sums = reinterpret_cast<v4e*>(lds_all);
+    auto at = [&](int g, int j, int i, int q) { return (((((g - 1) * NW + wave) * NI + j) * MI + i) * 4 + q) * 64 + lane; };
+    if (ks > 0) {
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            sums[at(ks, j, i, q)] =
+                v4e{acc[j][i][4 * q], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]};
+    }
+    __syncthreads();
+    if (ks == 0) {
+#pragma unroll
+      for (int g = 1; g < KS; ++g)
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+#pragma unroll
+          for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const v4e o = sums[at(g, j, i, q)];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[j][i][4 * q + e] += o[e];
+            }
+    }
+    __syncthreads();  // the sums are read before group 0's slabs overwrite them
+    if (ks > 0) return;
+  }
+
+  uint8_t* const wst = lds_all + wave * (T::SLABS * 32 * WPITCH);
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    uint8_t* const slab = wst + (i & (T::SLABS - 1)) * 32 * WPITCH;
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int cw = j * 32 + 8 * g + 4 * half;
+        const float b4[4] = {bf16_lo_to_f32(bv[j][g].x), bf16_hi_to_f32(bv[j][g].x), bf16_lo_to_f32(bv[j][g].y),
+                             bf16_hi_to_f32(bv[j][g].y)};
+        float y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (kI8) {
+            const float sw4[4] = {swv[j][g].x, swv[j][g].y, swv[j][g].z, swv[j][g].w};
+            y[e] = __fmul_rn(__fmul_rn(static_cast<float>(acc[j][i][4 * g + e]), sxv[i]), sw4[e]);
+          } else if constexpr (kFp8) {
+            y[e] = __fmul_rn(acc[j][i][4 * g + e], scale);
+          } else {
+            y[e] = acc[j][i][4 * g + e];
+          }
+          y[e] = __fadd_rn(y[e], b4[e]);
+          if constexpr (ACT != 0) {
+            const float r = __uint_as_float(pack_bf16x2_hw(y[e], 0.f) << 16);
+            y[e] = ACT == 1 ? silu(r) : gelu_tanh(r);
+          }
+        }
+        *reinterpret_cast<uint2*>(slab + l32 * WPITCH + cw * 2) =
+            make_uint2(pack_bf16x2_hw(y[0], y[1]), pack_bf16x2_hw(y[2], y[3]));
+      }
+    // the slab's rows are read back by other lanes of this wave: LDS executes a wave's accesses in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    constexpr int LPR = NI * 4;        // lanes of 8 columns per output row
+    constexpr int RPI = 64 / LPR;      // rows per store instruction
+    const int ch = lane % LPR;
+    const int gn = n0 + wn * NI * 32 + ch * 8;
+#pragma unroll
+    for (int it = 0; it < 32 / RPI; ++it) {
+      const int rr = it * RPI + lane / LPR;
+      const uint4 v = *reinterpret_cast<const uint4*>(slab + rr * WPITCH + ch * 16);
+      const int gm = m0 + (wm * MI + i) * 32 + rr;
+      if (gm < p.M && gn < p.N) {
+        uint16_t* dst = p.y + static_cast<int64_t>(gm) * p.ldy + gn;
+        if (p.vec16 && gn + 8 <= p.N) {
+          *reinterpret_cast<uint4*>(dst) = v;
+        } else {
+          *reinterpret_cast<uint2*>(dst) = make_uint2(v.x, v.y);
+          if (gn + 8 <= p.N) *reinterpret_cast<uint2*>(dst + 4) = make_uint2(v.z, v.w);
+        }
+      }
+    }
+  }
+}
+
+template <typename T, typename OP, int ACT>
+void launch_small(const SmallArgs& p, hipStream_t stream) {
+  const int64_t tiles = static_cast<int64_t>((p.M + T::BM - 1) / T::BM) * ((p.N + T::BN - 1) / T::BN);
+  const dim3 grid(static_cast<uint32_t>((tiles + NUM_XCD - 1) / NUM_XCD * NUM_XCD));
+  hipLaunchKernelGGL((gemm_small_kernel<T, OP, ACT>), grid, dim3(T::THREADS), 0, stream, p);
+}
+
+// The tiles.  In-workgroup split of K (KS) for the two small ones, whose time is the latency of a K step (about
+// 350-450 cycles whatever its bytes); e4m3 keeps one group, so that its fp32 sums keep the order they have in the
+// large tiles.
+template <typename OP>
+struct SmallTiles {
+  static constexpr bool split = !std::is_same<OP, OpFp8>::value;
+  using T0 = typename std::conditional<split, SmallTile<32, 64, 1, 2, 3, 4>, SmallTile<32, 64, 1, 2, 6>>::type;
+  using T1 = typename std::conditional<split, SmallTile<64, 64, 2, 2, 4, 2>, SmallTile<64, 64, 2, 2, 4>>::type;
+  using T2 = SmallTile<64, 128, 2, 4, 3>;
+  using T3 = SmallTile<128, 128, 2, 4, 4>;
+};
+
+// The tile of an M x N output with kb bytes of K, or -1 when `always` is false and the large tiles are the better
+// ones: the smallest tile that covers the output in one round of workgroups (one per CU), because a round's time
+// grows with the tile (int8, K = 1536 / 8960, us: 32 x 64 5.2 / 12.6, 64 x 64 5.7 / 15.4, 64 x 128 6.7 / 22.5,
+// 128 x 128 8.9 / 30.4, 128 x 256 11.5 / 40) and a second round costs more than the next tile up (512 x 1536 x 1536:
+// 32 x 64 in two rounds 9.2, 64 x 64 in one 6.0).  Past one round of 128 x 128 the 128 x 256 tile is ahead
+// (1560 x 4608 x 1536: 17.5 against 20.4).  A K of at most four steps is all launch, fill and stores: 64 x 128,
+// two workgroups per CU (4680 x 1536, K = 64 bf16: 8.4 against 10.5 / 39 us for 64 x 64 / 32 x 64).
+inline int pick_small(int M, int N, int kb, bool always) {
+  if (g_tile_policy >= 2) return g_tile_policy - 2;
+  const int64_t cus = device_cus();
+  auto tiles = [&](int bm, int bn) { return static_cast<int64_t>((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  if (always && kb <= 4 * BK) return 2;
+  if (tiles(32, 64) <= cus) return 0;
+  if (tiles(64, 64) <= cus) return 1;
+  if (tiles(64, 128) <= cus) return 2;
+  if (always || tiles(128, 128) <= cus) return 3;
+  return -1;
+}
+
+template <typename OP, int ACT>
+void launch_small(int tile, const SmallArgs& p, hipStream_t stream) {
+  using S = SmallTiles<OP>;
+  switch (tile) {
+    case 0: launch_small<typename S::T0, OP, ACT>(p, stream); break;
+    case 1: launch_small<typename S::T1, OP, ACT>(p, stream); break;
+    case 2: launch_small<typename S::T2, OP, ACT>(p, stream); break;
+    default: launch_small<typename S::T3, OP, ACT>(p, stream); break;
+  }
+}
+
+}  // namespace gemm
+}  // namespace wf

@@ -67,20 +67,15 @@
 #include <type_traits>
 #include <utility>
 
+#include "gemm_core.hpp"
 #include "launchers.hpp"
 #include "wf_common.hpp"
 
 namespace wf {
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v8i __attribute__((ext_vector_type(8)));
-typedef int v16i __attribute__((ext_vector_type(16)));
-typedef float v16f __attribute__((ext_vector_type(16)));
+using namespace gemm;
 
-constexpr int BK = 128;  // K bytes per step
-constexpr int GROUP_M = 8;
-constexpr int NUM_XCD = 8;
 // The per-column epilogue operands in LDS, past the stages: sw (fp32) at 0, the bias as it arrives (bf16)
 // at 1024 and converted to fp32 at 2048.
 constexpr int EPI_BYTES = 3072;
@@ -112,60 +107,6 @@ struct Tile {
 };
 using TileStd = Tile<128, 3>;
 using TileBig = Tile<256, 2>;
-// Word 3 of a raw (untyped, stride 0) buffer resource on gfx9-family parts:
-// DATA_FORMAT = 32 bit.  With it, offsets >= num_records read as zero.
-constexpr int kBufferRsrcWord3 = 0x00020000;
-constexpr int kOutOfRange = 0x7ffffff0;
-
-// int8 x int8 -> int32, K = 32 per MFMA (one 16-byte piece per lane).
-struct OpI8 {
-  static constexpr int SUB = 4;
-  static constexpr int PIECES = 1;
-  typedef v16i acc_t;
-  __device__ static acc_t mfma(const v4i* w, const v4i* a, acc_t c) {
-    return __builtin_amdgcn_mfma_i32_32x32x32_i8(w[0], a[0], c, 0, 0, 0);
-  }
-};
-// e4m3 x e4m3 -> fp32, K = 64 per MFMA (two 16-byte pieces per lane).  Zero
-// scale operands select the unscaled v_mfma_f32_32x32x64_f8f6f4; format 0
-// is OCP e4m3 for both operands.
-struct OpFp8 {
-  static constexpr int SUB = 2;
-  static constexpr int PIECES = 2;
-  typedef v16f acc_t;
-  __device__ static acc_t mfma(const v4i* w, const v4i* a, acc_t c) {
-    const v8i wv = __builtin_shufflevector(w[0], w[1], 0, 1, 2, 3, 4, 5, 6, 7);
-    const v8i av = __builtin_shufflevector(a[0], a[1], 0, 1, 2, 3, 4, 5, 6, 7);
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wv, av, c, 0, 0, 0, 0, 0, 0);
-  }
-};
-
-template <typename F, int... I>
-__device__ inline void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ inline void static_for(F&& f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-template <int V>
-using ic = std::integral_constant<int, V>;
-
-// s_waitcnt with vmcnt(VM), lgkmcnt(LGKM) (15 = no wait), expcnt unchanged.
-template <int VM, int LGKM>
-__device__ inline void wait_counts() {
-  static_assert(VM >= 0 && VM < 64 && LGKM >= 0 && LGKM < 16, "wait counts");
-  __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | 0x70 | (LGKM << 8));
-}
-
-__device__ inline void dma16(__amdgpu_buffer_rsrc_t rsrc, uint8_t* lds_block, int offset) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, lds_block, 16, offset, 0, 0, 0);
-}
-__device__ inline void dma4(__amdgpu_buffer_rsrc_t rsrc, uint8_t* lds_block, int offset) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, lds_block, 4, offset, 0, 0, 0);
-}
-
-
 // A rectangle of the output that one launch covers with its workgroup tile: rows [m0, m1), columns [n0, n1);
 // m0 and n0 lie on the launch's tile grid and every tile but those at M or N lies wholly inside.
 struct Rect {
@@ -599,25 +540,6 @@ void launch_kernel(const GemmArgs& p, bool bias, bool gelu, hipStream_t stream) 
     hipLaunchKernelGGL((gemm_w8a8_kernel<T, OP, false, false, ACC>), grid, block, 0, stream, p);
 }
 
-// Tile plan: -1 the cost model below; 0 / 1 force the 128- / 256-row tile for the whole output (settable only
-// in the instrumented libraries, for A/B runs).
-int g_tile_policy = -1;
-
-// Compute units of the current device (one workgroup per CU at a time), cached per device (host threads may
-// call concurrently; each stores the same value).
-int device_cus() {
-  static std::atomic<int> cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int v = cus[dev].load(std::memory_order_relaxed);
-  if (v == 0) {
-    int n = 0;
-    v = (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) ? n : 256;
-    cus[dev].store(v, std::memory_order_relaxed);
-  }
-  return v;
-}
-
 // Both tiles run one workgroup per CU, so a launch takes about ceil(tiles / CUs) rounds of its tile's time.
 // A 256-row tile holds twice the work of a 128-row tile and takes about kBigTileCost times as long (1.62-1.83
 // on the eight Wan-1.3B / 14B linears at 4680 tokens, int8 and e4m3 alike).  Plans: the 128-row tile
@@ -840,7 +762,7 @@ extern "C" int wf_gemm_set_phase_buffer(uint64_t* stamps) {
 // 128 x 256 tile over the whole output, 1 the 256 x 256 tile over the whole output).
 extern "C" int wf_gemm_set_tile_policy(int policy) {
   WF_REQUIRE(policy >= -1 && policy <= 1, WF_E_INVALID, "wf_gemm_set_tile_policy: policy %d not in -1..1", policy);
-  wf::g_tile_policy = policy;
+  wf::gemm::g_tile_policy = policy;
   return WF_OK;
 }
 #endif

@@ -111,6 +111,11 @@ __device__ inline float gelu_tanh(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
+// x * sigmoid(x) = x / (1 + e^-x), on the hardware exponential and reciprocal.
+__device__ inline float silu(float x) {
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x));
+}
+
 // ------------------------------------------------------- wave64 reductions
 // DPP controls (gfx9): quad_perm [1,0,3,2] = 0xB1, [2,3,0,1] = 0x4E,
 // row_half_mirror (lane i <-> 7-i within 8) = 0x141.

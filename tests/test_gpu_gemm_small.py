@@ -15,6 +15,7 @@ import torch
 
 from waveforcing_amd import _lib
 from waveforcing_amd.dit import gemm_bf16
+from waveforcing_amd.fp8 import gemm_fp8_pertensor, gemm_i8
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -87,3 +88,42 @@ def test_flags_and_shapes_still_refused():
         m, k, lda, n, ldy, flags = args
         with pytest.raises(RuntimeError):
             _lib.call("wf_gemm_bf16", a.data_ptr(), m, k, lda, w.data_ptr(), n, None, y.data_ptr(), ldy, flags, st)
+
+
+# 32 x 64 tiles, 64 x 64, 64 x 128, 128 x 128, and one shape past them, each off the tile's edges
+W8A8_SHAPES = [(1, 4, 16), (31, 60, 112), (33, 68, 144), (77, 1536, 8960), (300, 1540, 1552), (512, 1536, 1536),
+               (150, 5120, 5120), (513, 1500, 400), (780, 1536, 1536), (790, 1540, 272), (1560, 1536, 1536),
+               (2047, 1924, 656), (4680, 1536, 1536)]
+
+
+@pytest.mark.parametrize("gelu", [False, True])
+@pytest.mark.parametrize("M,N,K", W8A8_SHAPES)
+def test_gemm_i8_small_tiles_equal_the_large_ones(M, N, K, gelu):
+    """The same bits as the 128 x 256 tiles, which a call that asks for the int32 accumulators runs (checked
+    against the oracle on their own), with and without a bias and into strided rows."""
+    g = torch.Generator().manual_seed(M + 3 * N + K)
+    qx = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8).to(DEV)
+    qw = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8).to(DEV)
+    sx = (torch.rand(M, generator=g) * 0.01 + 1e-3).to(DEV)
+    sw = (torch.rand(N, generator=g) * 0.01 + 1e-3).to(DEV)
+    for b in (_rand((N,), 5), None):
+        acc = torch.empty((M, N), dtype=torch.int32, device=DEV)
+        ref = gemm_i8(qx, qw, sx, sw, b, gelu=gelu, acc_out=acc)
+        y = torch.full((M + 1, N + 4), 3.0, dtype=torch.bfloat16, device=DEV)
+        gemm_i8(qx, qw, sx, sw, b, gelu=gelu, out=y[:M, :N])
+        assert torch.equal(y[:M, :N].contiguous().view(torch.int16), ref.view(torch.int16))
+        assert bool((y[M:] == 3.0).all()) and bool((y[:, N:] == 3.0).all())
+
+
+@pytest.mark.parametrize("M,N,K", W8A8_SHAPES)
+def test_gemm_e4m3_small_tiles(M, N, K):
+    """Against the product of the codes in 64 bits, within the bound above."""
+    x, w, b = _rand((M, K), M + K), _rand((N, K), N + K), _rand((N,), 9)
+    a8, w8 = x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+    sa, sw = torch.tensor([0.0123], device=DEV), torch.tensor([0.0456], device=DEV)
+    got = gemm_fp8_pertensor(a8, w8, sa, sw, b).double()
+    s = float(sa) * float(sw)
+    a64, w64 = a8.float().double(), w8.float().double()
+    pre = (a64 @ w64.t()) * s + b.double()
+    bound = (K + 8) * 2.0 ** -23 * s * (a64.abs() @ w64.abs().t()) + (2.0 ** -8 + 2.0 ** -22) * pre.abs()
+    assert bool(((got - pre).abs() <= bound * 1.01 + 1e-30).all())

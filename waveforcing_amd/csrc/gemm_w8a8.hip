@@ -68,6 +68,7 @@
 #include <utility>
 
 #include "gemm_core.hpp"
+#include "gemm_small.hpp"
 #include "launchers.hpp"
 #include "wf_common.hpp"
 
@@ -613,6 +614,19 @@ Plan plan_tiles(int M, int N, int K) {
 template <typename OP>
 int launch(const GemmArgs& p0, bool bias, bool gelu, hipStream_t stream, const char* fn) {
   const bool acc = std::is_same<OP, OpI8>::value && p0.acc_out != nullptr;
+  // Outputs that one round of the small tiles covers (acc_out is only written by the large ones).
+  if (!acc && (g_tile_policy == -1 || g_tile_policy >= 2)) {
+    const int tile = pick_small(p0.M, p0.N, p0.K, false);
+    if (tile >= 0) {
+      const SmallArgs q{p0.a, p0.w, p0.sx, p0.sw, p0.bias, p0.y, p0.M, p0.N, p0.K, p0.K, p0.ldy, p0.vec16, 1};
+      constexpr int kGelu = std::is_same<OP, OpI8>::value ? 2 : 0;
+      if (gelu)
+        launch_small<OP, kGelu>(tile, q, stream);
+      else
+        launch_small<OP, 0>(tile, q, stream);
+      return check_launch(fn);
+    }
+  }
   const Plan plan = plan_tiles(p0.M, p0.N, p0.K);
   GemmArgs p = p0;
   if (plan.big_rects > 0) {
@@ -759,9 +773,9 @@ extern "C" int wf_gemm_set_phase_buffer(uint64_t* stamps) {
 #endif
 #if defined(WF_GEMM_PHASES) || defined(WF_GEMM_TILE_LAB)
 // Instrumented builds only: the tile plan of the following GEMM launches (-1 the product's plan, 0 the
-// 128 x 256 tile over the whole output, 1 the 256 x 256 tile over the whole output).
+// 128 x 256 tile over the whole output, 1 the 256 x 256 tile, 2 + i the small tile i).
 extern "C" int wf_gemm_set_tile_policy(int policy) {
-  WF_REQUIRE(policy >= -1 && policy <= 1, WF_E_INVALID, "wf_gemm_set_tile_policy: policy %d not in -1..1", policy);
+  WF_REQUIRE(policy >= -1 && policy <= 5, WF_E_INVALID, "wf_gemm_set_tile_policy: policy %d not in -1..5", policy);
   wf::gemm::g_tile_policy = policy;
   return WF_OK;
 }

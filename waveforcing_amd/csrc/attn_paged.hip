@@ -42,6 +42,17 @@
 // A wave issues a VALU instruction at most every ~8 cycles on gfx950, so
 // the vector work only hides when it sits between the wave's own MFMAs.
 //
+// Few queries (FEW): a grid of 256-query workgroups that leaves CUs idle is split finer instead.  Four waves own
+// 32 queries each (or fewer of them do) and four other waves stage for all, so a query wave shares its SIMD with a
+// light mate and issues nothing but its scores, softmax and PV: a tile takes 0.9-1.1 us instead of 1.5-1.8 us,
+// for at most half the queries.  The staging waves keep two further tiles in flight in registers.  Every query's
+// arithmetic is that of the 256-query form, so its output bits do not depend on the split.  1560 queries x 12
+// heads x 10920 keys, 84 -> 204 workgroups: exact 270 -> 157 us, quantized QK 310 -> 183, fp8 PV 306 -> 194; 300
+// queries x 5000 keys 128 -> 72, 147 -> 81, 145 -> 86; 48 queries x 3000 keys 77 -> 44, 80 -> 50, 83 -> 53;
+// dense 1560 x 10920 256 -> 154.  What bounds it now is one wave's issue rate (a VALU every 5-6.5 cycles, ~210
+// instructions per tile); running the next tile's score MFMAs under the softmax there gained 7 % (dense,
+// quantized QK) and lost 6 % (exact), so one body serves both splits.
+//
 // Softmax in base 2 with the scale folded into one FMA per score, and lazy
 // rescaling: a query's running maximum used in the exponent is raised only
 // when its tile maximum exceeds it by more than kTau (log2 units), so
@@ -56,6 +67,7 @@
 
 #include "fastdiv.hpp"
 #include "fp8_codec.hpp"
+#include "gemm_core.hpp"
 #include "wf_common.hpp"
 
 namespace wf {
@@ -119,6 +131,7 @@ struct AttnArgs {
   int Lq, H, n_kv, n_table, page_tokens, pool_pages;
   FastDiv page_div;
   float qk_scale;  // softmax scale * log2(e)
+  int bq;          // queries per workgroup: BQ, or 32..128 with FEW
 };
 
 // Two fp32 -> packed bf16x2, round to nearest even (v_cvt_pk_bf16_f32).
@@ -189,10 +202,11 @@ __device__ inline float pair_sum(float v) {
 // scale s_v goes into P, each query's 64 values p_k s_v,k of a tile are rounded to e4m3 after division by
 // 2^E, the smallest power of two that brings their maximum to <= 448 (the same rule as the queries'), and 2^E
 // is the MFMA's block scale of that query's column.  The row sum stays the fp32 sum of the unrounded p_k.
-template <bool DENSE, bool QK8, bool PV8>
+template <bool DENSE, bool QK8, bool PV8, bool FEW>
 __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) {
   static_assert(!(DENSE && QK8), "the quantized-QK form reads FP8 pages");
   static_assert(!PV8 || QK8, "the fp8-PV form extends the quantized-QK form");
+  static_assert(WAVES == 8, "FEW: four query waves and four staging waves");
   constexpr int kStage = PV8 ? STAGE_PV8 : QK8 ? STAGE8 : STAGE;
   constexpr int kVOff = QK8 ? K8_TILE : K_TILE;              // V rows within a stage
   constexpr int kSOff = K8_TILE + (PV8 ? V8_TILE : V_TILE);  // u_k within a stage (QK8)
@@ -202,27 +216,27 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31;
   const int half = lane >> 5;
   // Work item w = head * q_tiles + q_tile.  Workgroups are dealt to the 8
   // XCDs round-robin (blockIdx % 8); each XCD gets a contiguous range of
   // work items, so the query tiles of one head share that head's K/V tiles
   // in one L2.
-  const int q_tiles = (p.Lq + BQ - 1) / BQ;
+  const int bq = FEW ? p.bq : BQ;
+  const int q_tiles = (p.Lq + bq - 1) / bq;
   const int n_items = q_tiles * p.H;
   const int per_xcd = (n_items + 7) / 8;
   const int w_item = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
   if (w_item >= n_items) return;
   const int h = w_item / q_tiles;
-  const int q0 = (w_item % q_tiles) * BQ;
+  const int q0 = (w_item % q_tiles) * bq;
 
   // ---- staging role: key skey of the tile, d = 16 * schunk .. + 15 ---------
-  const int skey = tid >> 3;
+  // (FEW: waves 4..7 stage, keys skey and skey + 32)
+  const int skey = FEW ? (tid >> 3) & 31 : tid >> 3;
   const int schunk = tid & 7;
   const int HD = p.H * D;
-  const int lane_co = skey * HD + schunk * 16;  // this thread's key row within a page, codes
-  const int lane_so = skey * 4;                 // and scales
 
   __amdgpu_buffer_rsrc_t rk, rv, rsk, rsv;
   if constexpr (DENSE) {
@@ -243,8 +257,11 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
   }
 
   // One tile's staging registers: 16 codes (or 2 x 8 bf16) of K and of V, and the scales.
-  u32x4 sk0, sv0, sk1, sv1;
-  float ssk = 0.f, ssv = 0.f;
+  struct Staged {
+    u32x4 k0, v0, k1, v1;
+    float sk, sv;
+  };
+  Staged sreg;
 
   // Page cursor of a tile (uniform across the workgroup): keys [0, split) of a tile starting at key t0 sit
   // on the physical page of logical page lp from row r0 (split = page_tokens - r0), keys [split, 64) on
@@ -304,65 +321,65 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
   };
 
   // Issue the loads of the tile starting at key t0 (cursor c).
-  auto load_tile = [&](int t0, const Cursor& c) {
+  auto load_tile = [&](int t0, const Cursor& c, Staged& r, int skey) {
     if constexpr (DENSE) {
       (void)c;
       const int key = min(t0 + skey, p.n_kv);
       const uint32_t off = static_cast<uint32_t>((key * static_cast<int>(p.ldkv) + h * D + schunk * 16) * 2) +
                            (key < p.n_kv ? 0u : static_cast<uint32_t>(kOutOfRange));
-      sk0 = __builtin_amdgcn_raw_buffer_load_b128(rk, static_cast<int>(off), 0, 0);
-      sk1 = __builtin_amdgcn_raw_buffer_load_b128(rk, static_cast<int>(off + 16), 0, 0);
-      sv0 = __builtin_amdgcn_raw_buffer_load_b128(rv, static_cast<int>(off), 0, 0);
-      sv1 = __builtin_amdgcn_raw_buffer_load_b128(rv, static_cast<int>(off + 16), 0, 0);
+      r.k0 = __builtin_amdgcn_raw_buffer_load_b128(rk, static_cast<int>(off), 0, 0);
+      r.k1 = __builtin_amdgcn_raw_buffer_load_b128(rk, static_cast<int>(off + 16), 0, 0);
+      r.v0 = __builtin_amdgcn_raw_buffer_load_b128(rv, static_cast<int>(off), 0, 0);
+      r.v1 = __builtin_amdgcn_raw_buffer_load_b128(rv, static_cast<int>(off + 16), 0, 0);
     } else {
       // Branch-free: keys past n_kv are pushed out of range like an invalid page.
       const bool first = skey < p.page_tokens - c.r0;
       const uint32_t lm = 0u - static_cast<uint32_t>(skey < p.n_kv - t0);   // all ones for keys before n_kv
       const uint32_t lfar = static_cast<uint32_t>(kOutOfRange) & ~lm;
-      const uint32_t co = (((first ? c.cb0 : c.cb1) + static_cast<uint32_t>(lane_co)) & lm) | lfar;
-      const uint32_t so = (((first ? c.sb0 : c.sb1) + static_cast<uint32_t>(lane_so)) & lm) | lfar;
-      sk0 = __builtin_amdgcn_raw_buffer_load_b128(rk, static_cast<int>(co), 0, 0);
-      sv0 = __builtin_amdgcn_raw_buffer_load_b128(rv, static_cast<int>(co), 0, 0);
-      ssk = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsk, static_cast<int>(so), 0, 0));
-      ssv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsv, static_cast<int>(so), 0, 0));
+      const uint32_t co = (((first ? c.cb0 : c.cb1) + static_cast<uint32_t>(skey * HD + schunk * 16)) & lm) | lfar;
+      const uint32_t so = (((first ? c.sb0 : c.sb1) + static_cast<uint32_t>(skey * 4)) & lm) | lfar;
+      r.k0 = __builtin_amdgcn_raw_buffer_load_b128(rk, static_cast<int>(co), 0, 0);
+      r.v0 = __builtin_amdgcn_raw_buffer_load_b128(rv, static_cast<int>(co), 0, 0);
+      r.sk = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsk, static_cast<int>(so), 0, 0));
+      r.sv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsv, static_cast<int>(so), 0, 0));
     }
   };
 
   // The staged tile as bf16 [key][d] row pieces (registers only), and their
   // write into LDS stage `buf`.
-  auto dequant_tile = [&](uint4* out) {
+  auto dequant_tile = [&](const Staged& r, uint4* out) {
     if constexpr (PV8) {
       // K and V codes as they are, u_k and the V scale alongside
-      out[0] = make_uint4(sk0[0], sk0[1], sk0[2], sk0[3]);
-      out[1] = make_uint4(__builtin_bit_cast(uint32_t, __fmul_rn(ssk, p.qk_scale)), __builtin_bit_cast(uint32_t, ssv),
+      out[0] = make_uint4(r.k0[0], r.k0[1], r.k0[2], r.k0[3]);
+      out[1] = make_uint4(__builtin_bit_cast(uint32_t, __fmul_rn(r.sk, p.qk_scale)), __builtin_bit_cast(uint32_t, r.sv),
                           0u, 0u);
-      out[2] = make_uint4(sv0[0], sv0[1], sv0[2], sv0[3]);
+      out[2] = make_uint4(r.v0[0], r.v0[1], r.v0[2], r.v0[3]);
     } else if constexpr (QK8) {
       // K codes as they are, the key's exponent factor u_k = s_k * softmax scale * log2(e) alongside; V as in
       // the bf16 form
-      out[0] = make_uint4(sk0[0], sk0[1], sk0[2], sk0[3]);
-      out[1] = make_uint4(__builtin_bit_cast(uint32_t, __fmul_rn(ssk, p.qk_scale)), 0u, 0u, 0u);
-      const uint2 e = dequant4_bf16(sv0[0], ssv), f = dequant4_bf16(sv0[1], ssv);
-      const uint2 g = dequant4_bf16(sv0[2], ssv), i = dequant4_bf16(sv0[3], ssv);
+      out[0] = make_uint4(r.k0[0], r.k0[1], r.k0[2], r.k0[3]);
+      out[1] = make_uint4(__builtin_bit_cast(uint32_t, __fmul_rn(r.sk, p.qk_scale)), 0u, 0u, 0u);
+      const uint2 e = dequant4_bf16(r.v0[0], r.sv), f = dequant4_bf16(r.v0[1], r.sv);
+      const uint2 g = dequant4_bf16(r.v0[2], r.sv), i = dequant4_bf16(r.v0[3], r.sv);
       out[2] = make_uint4(e.x, e.y, f.x, f.y);
       out[3] = make_uint4(g.x, g.y, i.x, i.y);
     } else if constexpr (DENSE) {
-      out[0] = make_uint4(sk0[0], sk0[1], sk0[2], sk0[3]);
-      out[1] = make_uint4(sk1[0], sk1[1], sk1[2], sk1[3]);
-      out[2] = make_uint4(sv0[0], sv0[1], sv0[2], sv0[3]);
-      out[3] = make_uint4(sv1[0], sv1[1], sv1[2], sv1[3]);
+      out[0] = make_uint4(r.k0[0], r.k0[1], r.k0[2], r.k0[3]);
+      out[1] = make_uint4(r.k1[0], r.k1[1], r.k1[2], r.k1[3]);
+      out[2] = make_uint4(r.v0[0], r.v0[1], r.v0[2], r.v0[3]);
+      out[3] = make_uint4(r.v1[0], r.v1[1], r.v1[2], r.v1[3]);
     } else {
-      const uint2 a = dequant4_bf16(sk0[0], ssk), b = dequant4_bf16(sk0[1], ssk);
-      const uint2 c = dequant4_bf16(sk0[2], ssk), d = dequant4_bf16(sk0[3], ssk);
+      const uint2 a = dequant4_bf16(r.k0[0], r.sk), b = dequant4_bf16(r.k0[1], r.sk);
+      const uint2 c = dequant4_bf16(r.k0[2], r.sk), d = dequant4_bf16(r.k0[3], r.sk);
       out[0] = make_uint4(a.x, a.y, b.x, b.y);
       out[1] = make_uint4(c.x, c.y, d.x, d.y);
-      const uint2 e = dequant4_bf16(sv0[0], ssv), f = dequant4_bf16(sv0[1], ssv);
-      const uint2 g = dequant4_bf16(sv0[2], ssv), i = dequant4_bf16(sv0[3], ssv);
+      const uint2 e = dequant4_bf16(r.v0[0], r.sv), f = dequant4_bf16(r.v0[1], r.sv);
+      const uint2 g = dequant4_bf16(r.v0[2], r.sv), i = dequant4_bf16(r.v0[3], r.sv);
       out[2] = make_uint4(e.x, e.y, f.x, f.y);
       out[3] = make_uint4(g.x, g.y, i.x, i.y);
     }
   };
-  auto write_tile = [&](int buf, const uint4* v) {
+  auto write_tile = [&](int buf, const uint4* v, int skey) {
     if constexpr (PV8) {
       uint8_t* sb = lds + buf * kStage;
       *reinterpret_cast<uint4*>(sb + skey * KP8 + schunk * 16) = v[0];
@@ -384,11 +401,55 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
     dv[0] = v[2];
     dv[1] = v[3];
   };
-  auto store_tile = [&](int buf) {
+  auto store_tile = [&](int buf, const Staged& r, int skey) {
     uint4 v[4];
-    dequant_tile(v);
-    write_tile(buf, v);
+    dequant_tile(r, v);
+    write_tile(buf, v, skey);
   };
+
+  const int n_tiles = (p.n_kv + BKV - 1) / BKV;
+  if constexpr (FEW) {
+    // Waves 4..7 stage every tile; waves 0..3 own 32 queries each, and those past the workgroup's queries only
+    // keep the barriers.  Two tiles are in flight in registers while a third is being written.
+    if (n_tiles > 0 && wave >= 4) {
+      Staged r[2][2];
+      Cursor cu = cursor_at(0);
+      // (the fences keep the loads in tile order, so that a tile's wait leaves the next tile's in flight)
+      auto load = [&](int t, Staged* x) {
+        load_tile(t * BKV, cu, x[0], skey);
+        load_tile(t * BKV, cu, x[1], skey + 32);
+        cu = cursor_next(cu, (t + 1) * BKV);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto store = [&](int t, Staged* x) {
+        store_tile(t & 1, x[0], skey);
+        store_tile(t & 1, x[1], skey + 32);
+      };
+      load(0, r[0]);
+      load(1, r[1]);
+      store(0, r[0]);
+      load(2, r[0]);
+      __syncthreads();
+      // iteration it: tile it is computed, tile it + 1 written, tile it + 3 loaded.  No exit between the two
+      // halves: on a path from the first half back to the top the compiler would wait for every load there.
+      int it = 0;
+      for (; it + 1 < n_tiles; it += 2) {
+        store(it + 1, r[1]);
+        load(it + 3, r[1]);
+        __syncthreads();
+        store(it + 2, r[0]);
+        load(it + 4, r[0]);
+        __syncthreads();
+      }
+      if (it < n_tiles) __syncthreads();  // an odd count's last tile: nothing left to stage
+      return;
+    }
+    if (wave >= 4 || 32 * wave >= bq || q0 + 32 * wave >= p.Lq) {
+      if (n_tiles > 0)
+        for (int it = 0; it <= n_tiles; ++it) __syncthreads();
+      return;
+    }
+  }
 
   // ---- Q^T fragments for this wave's 32 queries (kept for the whole kernel)
   v8bf qf[QK8 ? 1 : 8];
@@ -487,7 +548,6 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
   float neg_mc = 0.f;       // -m_use * c
   float l_run = 0.f;        // this half's row sum (its 32 of every 64 keys)
 
-  const int n_tiles = (p.n_kv + BKV - 1) / BKV;
   Cursor cur_next{};  // the cursor of the tile loaded in the next iteration
 
   // One tile: scores with the staging of the next tile (into the other stage,
@@ -521,7 +581,7 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
 #pragma unroll
         for (int g = 0; g < 4; ++g)
           skv[b][g] = *reinterpret_cast<const float4*>(st + kSOff + 4 * (32 * b + 8 * g + 4 * half));
-      dequant_tile(nxt);
+      if constexpr (!FEW) dequant_tile(sreg, nxt);
 #pragma unroll
       for (int b = 0; b < 2; ++b) s[b] = v16f{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
@@ -533,7 +593,7 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // then 1 MFMA
-        __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);  // and 8 VALU, alternating
+        if constexpr (!FEW) __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);  // and 8 VALU, alternating
       }
     } else {
       // K fragments of the tile, all in flight before the first MFMA.
@@ -545,7 +605,7 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
           kf[b][ks] = __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4*>(st + k_lane + b * 32 * KP + ks * 32));
       // S^T = K Q^T for 2 blocks of 32 keys, with the next tile's dequantization
       // (registers only) between the MFMAs.
-      dequant_tile(nxt);
+      if constexpr (!FEW) dequant_tile(sreg, nxt);
 #pragma unroll
       for (int b = 0; b < 2; ++b) s[b] = v16f{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
@@ -556,14 +616,16 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // then 1 MFMA
-        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // and 4 VALU, alternating
+        if constexpr (!FEW) __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // and 4 VALU, alternating
       }
     }
     // the next tile into the other stage (freed by the last barrier), the
     // loads of the one after, and this tile's V^T operands (in flight
     // during the softmax).
-    write_tile(cur ^ 1, nxt);
-    load_tile((it + 2) * BKV, cur_next);
+    if constexpr (!FEW) {
+      write_tile(cur ^ 1, nxt, skey);
+      load_tile((it + 2) * BKV, cur_next, sreg, skey);
+    }
     v8bf vf[PV8 ? 1 : 4][4];
     v8i vf8[4];
     float4 svv[2][4];  // PV8: s_v of the lane's keys 32 b + 8 g + 4 half + 0..3
@@ -704,7 +766,7 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
 #pragma unroll
       for (int db = 0; db < 4; ++db)
         o[db] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf8[db], pb, o[db], 0, 0, 0, 127, 0, 127 + E);
-      cur_next = cursor_next(cur_next, (it + 3) * BKV);
+      if constexpr (!FEW) cur_next = cursor_next(cur_next, (it + 3) * BKV);
       __syncthreads();
       return;
     }
@@ -732,17 +794,19 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
 #pragma unroll
       for (int db = 0; db < 4; ++db) o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[t][db], pf, o[db], 0, 0, 0);
     }
-    cur_next = cursor_next(cur_next, (it + 3) * BKV);
+    if constexpr (!FEW) cur_next = cursor_next(cur_next, (it + 3) * BKV);
     __syncthreads();
   };
 
   if (n_tiles > 0) {
-    cur_next = cursor_at(0);
-    load_tile(0, cur_next);
-    store_tile(0);
-    cur_next = cursor_next(cur_next, BKV);
-    load_tile(BKV, cur_next);
-    cur_next = cursor_next(cur_next, 2 * BKV);
+    if constexpr (!FEW) {
+      cur_next = cursor_at(0);
+      load_tile(0, cur_next, sreg, skey);
+      store_tile(0, sreg, skey);
+      cur_next = cursor_next(cur_next, BKV);
+      load_tile(BKV, cur_next, sreg, skey);
+      cur_next = cursor_next(cur_next, 2 * BKV);
+    }
     __syncthreads();
     for (int it = 0; it + 1 < n_tiles; ++it) body(it, std::false_type{});
     body(n_tiles - 1, std::true_type{});
@@ -774,11 +838,41 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
 
 }  // namespace
 
+// Queries per workgroup: the split whose rounds of workgroups (one per CU) take least.  Cost of a round against
+// the 128-query split's, measured per tile over the four forms: 256 queries 1.55-1.67, 96 queries 0.92-1.0, 64 and
+// 32 queries 0.90-0.97 (fewer query waves contend for LDS).  4680 queries x 12 heads: 228 workgroups of 256 in one
+// round (22.9 us over 512 keys) against 444 of 128 in two (27.7 us); 1560 x 40 heads x 10920 keys: 280 of 256 in
+// two rounds 577 us, 520 of 128 in three 491 us, 680 of 96 in three 476 us.
+int pick_queries(int64_t lq, int n_heads, int64_t n_kv) {
+  // the staging waves index up to four tiles past the last
+  if (n_kv >= (1ll << 31) - 8 * BKV) return BQ;
+  static constexpr struct {
+    int bq;
+    double cost;
+  } kSplits[] = {{BQ, 1.6}, {128, 1.0}, {96, 0.95}, {64, 0.94}, {32, 0.92}};
+  const int64_t cus = gemm::device_cus();
+  int best = BQ;
+  double best_cost = 0;
+  for (const auto& sp : kSplits) {
+    const int64_t items = (lq + sp.bq - 1) / sp.bq * n_heads;
+    const double cost = sp.cost * static_cast<double>((items + cus - 1) / cus);
+    if (sp.bq == BQ || cost < best_cost) {
+      best = sp.bq;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 template <bool DENSE, bool QK8, bool PV8>
-int launch_attn(const AttnArgs& p, int64_t lq, int n_heads, hipStream_t stream) {
-  const int64_t items = (lq + BQ - 1) / BQ * n_heads;
+int launch_attn(AttnArgs p, int64_t lq, int n_heads, hipStream_t stream) {
+  p.bq = pick_queries(lq, n_heads, p.n_kv);
+  const int64_t items = (lq + p.bq - 1) / p.bq * n_heads;
   const dim3 grid(static_cast<uint32_t>((items + 7) / 8 * 8));
-  hipLaunchKernelGGL((attn_paged_fp8_kernel<DENSE, QK8, PV8>), grid, dim3(THREADS), 0, stream, p);
+  if (p.bq == BQ)
+    hipLaunchKernelGGL((attn_paged_fp8_kernel<DENSE, QK8, PV8, false>), grid, dim3(THREADS), 0, stream, p);
+  else
+    hipLaunchKernelGGL((attn_paged_fp8_kernel<DENSE, QK8, PV8, true>), grid, dim3(THREADS), 0, stream, p);
   return check_launch(DENSE  ? "wf_attn_dense_bf16"
                       : PV8 ? "wf_attn_paged_fp8_qkpv8"
                       : QK8 ? "wf_attn_paged_fp8_qk8"

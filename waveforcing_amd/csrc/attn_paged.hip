@@ -47,8 +47,8 @@
 // light mate and issues nothing but its scores, softmax and PV: a tile takes 0.9-1.1 us instead of 1.5-1.8 us,
 // for at most half the queries.  The staging waves keep two further tiles in flight in registers.  Every query's
 // arithmetic is that of the 256-query form, so its output bits do not depend on the split.  1560 queries x 12
-// heads x 10920 keys, 84 -> 204 workgroups: exact 270 -> 157-172 us, quantized QK 310 -> 183, fp8 PV 306 -> 194;
-// 300 queries x 5000 keys 128 -> 72, 147 -> 81, 145 -> 86; 48 queries x 3000 keys 77 -> 44, 80 -> 50, 83 -> 53;
+// heads x 10920 keys, 84 -> 204 workgroups: exact 270 -> 157 us, quantized QK 310 -> 183, fp8 PV 306 -> 194; 300
+// queries x 5000 keys 128 -> 72, 147 -> 81, 145 -> 86; 48 queries x 3000 keys 77 -> 44, 80 -> 50, 83 -> 53;
 // dense 1560 x 10920 256 -> 154.  What bounds it now is one wave's issue rate (a VALU every 5-6.5 cycles, ~210
 // instructions per tile); running the next tile's score MFMAs under the softmax there gained 7 % (dense,
 // quantized QK) and lost 6 % (exact), so one body serves both splits.
@@ -60,15 +60,6 @@
 // divides by the row sum taken against the same maximum, so the result is
 // unchanged.  The decision is per query, so every output row depends only on
 // its own query and the context.
-// The quantized-QK form forms the exponents first and takes their exact
-// maximum instead of a bound of it (a maximum of the scores and one of u_k):
-// 20 VALU instructions per tile fewer, and with heavy-tailed K, where the
-// bound lies far above the scores, most rescales: 4680 queries x 12 heads x
-// 37440 keys 1053 -> 986 us, 40 heads x 9360 keys 909 -> 853, 1560 x 12 x 10920
-// 184 -> 165, 300 x 5000 81 -> 73.  Leaving the maximum out until the weights
-// of a tile sum too high measured 916, 781, 137 and 59 us, but 0.3-1.8 % more
-// error against 64 bits (the largest weight is then not exactly 1); the exact
-// form gained nothing from that.
 // K stays exactly bf16(code * s): with heavy-tailed K the scores reach
 // magnitudes where any further rounding of K (e.g. folding the scale into
 // it) moves P by percents.
@@ -203,8 +194,10 @@ __device__ inline float pair_sum(float v) {
 // pages are used as they are, and S^T = K_codes Q_codes^T runs on the fp8 matrix cores
 // (v_mfma_scale_f32_32x32x64_f8f6f4), which apply 2^e_q to each query's column as its block scale.  The
 // staging stores u_k = s_k * softmax scale * log2(e) per key, the same for every query, so a score's exponent
-// is one FMA, s'' u_k - m (fp8 PV: the tile's maximum is bounded by max s'' * max u_k, exact maxima only in the
-// rare rescale).  V and P stay exact as in the bf16 form.
+// is one FMA, s'' u_k - m; the tile's maximum is bounded by max s'' * max u_k (exact maxima only in the rare
+// rescale).  V and P stay exact as in the bf16 form.  (Exponents before their exact maximum instead of the bound:
+// with heavy-tailed K, where the bound fires in most tiles, 4680 queries x 12 heads x 37440 keys 1053 -> 986 us; but
+// with N(0, 1) K 921 -> 963 and 2700 x 12 x 10920 263 -> 294, since the 32 FMAs then stand outside the PV MFMAs.)
 //
 // PV8 (with QK8): the fp8-PV form, the counterpart of the fp8 P.V product of the reference's SageAttention
 // backend.  V stays as the pages' codes in LDS and O^T += V^T P^T runs on the fp8 matrix cores too: the key
@@ -636,15 +629,6 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
       load_tile((it + 2) * BKV, cur_next, sreg, skey);
     }
     v8bf vf[PV8 ? 1 : 4][4];
-    auto read_v = [&](int t) {
-#pragma unroll
-      for (int db = 0; db < 4; ++db) {
-        const uint8_t* va = st + v_lane + (16 * t) * VP + db * 64;
-        const v4s lo = read_tr(va);
-        const v4s hi = read_tr(va + 8 * VP);
-        vf[t][db] = __builtin_bit_cast(v8bf, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-      }
-    };
     v8i vf8[4];
     float4 svv[2][4];  // PV8: s_v of the lane's keys 32 b + 8 g + 4 half + 0..3
     if constexpr (PV8) {
@@ -661,7 +645,14 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
           svv[b][g] = *reinterpret_cast<const float4*>(st + kVSOff + 4 * (32 * b + 8 * g + 4 * half));
     } else {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) read_v(t);
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int db = 0; db < 4; ++db) {
+          const uint8_t* va = st + v_lane + (16 * t) * VP + db * 64;
+          const v4s lo = read_tr(va);
+          const v4s hi = read_tr(va + 8 * VP);
+          vf[t][db] = __builtin_bit_cast(v8bf, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
     }
 
     // QK8: u_k of the lane's 32 keys as an array (element 4 g + e of block b), 1 for keys past n_kv (whose
@@ -691,73 +682,44 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
             if constexpr (QK8) u[b][4 * g + e] = past ? 1.0f : u[b][4 * g + e];
           }
     }
-    if constexpr (QK8 && !PV8) {
-      // The exponents x = s'' u_k - m (in s) before their maximum: a query's m is its exact running maximum, and only
-      // a tile that raises it for one of the wave's queries pays for the change (x, O and the row sum move by the
-      // difference; the raising key's weight is exactly 1).
+    float mt = -INFINITY;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) mt = fmaxf(mt, s[b][e]);
+    if constexpr (QK8) {
+      // an upper bound of the half's largest exponent s'' u_k: max s'' times the largest u_k when max s'' >= 0,
+      // else 0 (every exponent is negative); the exact maximum is taken only when the bound asks for a rescale
+      float um = 0.f;
 #pragma unroll
       for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) s[b][e] = fmaf(s[b][e], u[b][e], neg_mc);
-      float mt = -INFINITY;
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) mt = fmaxf(mt, s[b][e]);
-      mt = pair_max(mt);
-      if (it == 0 || __ballot(mt > 0.f)) {
-        float d = it == 0 ? mt : fmaxf(mt, 0.f);
-        if (d == -INFINITY) d = 0.f;
-        const float alpha = it == 0 ? 0.f : __builtin_amdgcn_exp2f(-d);
+        for (int e = 0; e < 16; ++e) um = fmaxf(um, u[b][e]);
+      mt = mt >= 0.f ? mt * um : 0.f;
+    }
+    mt = pair_max(mt);
+    // exponents in base 2: p = 2^(c * (s - m_use)), c = softmax_scale * log2(e) >= 0 (QK8: 2^(s'' u_k - m_use)).
+    // Each query decides for itself (the wave only branches when one of its queries rescales), so a query's
+    // output does not depend on which queries share its wave.
+    const bool fire = mt > m_thr;
+    if (__ballot(fire)) {
+      if constexpr (QK8) {
+        float ex = -INFINITY;
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
-          for (int e = 0; e < 16; ++e) s[b][e] -= d;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] *= alpha;
-        l_run *= alpha;
-        neg_mc -= d;
+          for (int e = 0; e < 16; ++e) ex = fmaxf(ex, s[b][e] * u[b][e]);
+        mt = pair_max(ex);
       }
-    } else {
-      float mt = -INFINITY;
+      const float m_new = fire ? fmaxf(m_use, mt) : m_use;
+      const float alpha =
+          !fire ? 1.f : (m_use == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(c * (m_use - m_new));
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) mt = fmaxf(mt, s[b][e]);
-      if constexpr (PV8) {
-        // an upper bound of the half's largest exponent s'' u_k: max s'' times the largest u_k when max s'' >= 0,
-        // else 0 (every exponent is negative); the exact maximum is taken only when the bound asks for a rescale
-        float um = 0.f;
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) um = fmaxf(um, u[b][e]);
-        mt = mt >= 0.f ? mt * um : 0.f;
-      }
-      mt = pair_max(mt);
-      // exponents in base 2: p = 2^(c * (s - m_use)), c = softmax_scale * log2(e) >= 0 (QK8: 2^(s'' u_k - m_use)).
-      // Each query decides for itself (the wave only branches when one of its queries rescales), so a query's
-      // output does not depend on which queries share its wave.
-      const bool fire = mt > m_thr;
-      if (__ballot(fire)) {
-        if constexpr (PV8) {
-          float ex = -INFINITY;
-#pragma unroll
-          for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) ex = fmaxf(ex, s[b][e] * u[b][e]);
-          mt = pair_max(ex);
-        }
-        const float m_new = fire ? fmaxf(m_use, mt) : m_use;
-        const float alpha =
-            !fire ? 1.f : (m_use == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(c * (m_use - m_new));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] *= alpha;
-        l_run *= alpha;
-        m_use = m_new;
-        m_thr = m_new + kTau / c;
-        neg_mc = (m_new == -INFINITY) ? 0.f : -m_new * c;
-      }
+      for (int i = 0; i < 4; ++i) o[i] *= alpha;
+      l_run *= alpha;
+      m_use = m_new;
+      m_thr = m_new + kTau / c;
+      neg_mc = (m_new == -INFINITY) ? 0.f : -m_new * c;
     }
     if constexpr (PV8) {
       // p_k (row sum) and p_k s_v,k; their maximum over the query's 64 keys (both halves) sets 2^E; the
@@ -820,8 +782,8 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         if constexpr (QK8) {
-          pv[e] = __builtin_amdgcn_exp2f(s[b][4 * g0 + e]);
-          pv[4 + e] = __builtin_amdgcn_exp2f(s[b][4 * g0 + 4 + e]);
+          pv[e] = __builtin_amdgcn_exp2f(fmaf(s[b][4 * g0 + e], u[b][4 * g0 + e], neg_mc));
+          pv[4 + e] = __builtin_amdgcn_exp2f(fmaf(s[b][4 * g0 + 4 + e], u[b][4 * g0 + 4 + e], neg_mc));
         } else {
           pv[e] = __builtin_amdgcn_exp2f(fmaf(s[b][4 * g0 + e], c, neg_mc));
           pv[4 + e] = __builtin_amdgcn_exp2f(fmaf(s[b][4 * g0 + 4 + e], c, neg_mc));

@@ -438,7 +438,9 @@ int wf_qk_norm_rope_kv_pack(void* q, int64_t ld_q, const void* norm_q,
 /* bf16 GEMM y[m][n] = act_out(bf16(sum_k act_in(a[m,k]) * w[n,k] + bias[n]))
  * with fp32 accumulation: a [m][k] (row stride lda), w [n][k] dense (nn.Linear
  * layout), bias bf16 [n] or NULL, y bf16 (row stride ldy).  k, lda % 8 == 0;
- * n, ldy % 4 == 0; a, w 16-byte and y 8-byte aligned.  The bf16 linears of
+ * n, ldy % 4 == 0; a, w 16-byte and y 8-byte aligned.  The sum of an output
+ * runs in one order whatever the sizes, so a row of y has the same bits in
+ * any call.  The bf16 linears of
  * the Wan DiT outside its blocks: the text embedding (Linear, GELU(tanh),
  * Linear), the time embedding (Linear, SiLU, Linear), the time projection
  * (SiLU, Linear), the head's Linear, and the patch embedding over

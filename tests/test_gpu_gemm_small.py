@@ -1,9 +1,9 @@
 """GPU parity of the small-output GEMM kernels at the edges of their tiles and of the rules that choose them.
 
 wf_gemm_bf16: the few-row kernel (1-16 rows; to 64 with SiLU on the input), the LDS tiles of gemm_small.hpp (32 x 64
-and 64 x 64 with K split over groups of waves, 64 x 128, 128 x 128) and the direct kernel behind them; sizes one
-off a tile, K tails inside a 64-element step, rows and columns past the end, strided A and y, a bias that is only
-2-byte aligned, no bias.
+and 64 x 64 with loading waves of their own, 64 x 128, 128 x 128) and the direct kernel behind them, which all give
+a row the same bits; sizes one off a tile, K tails inside a 64-element step, rows and columns past the end,
+strided A and y, a bias that is only 2-byte aligned, no bias.
 
 Bound per element, against the product in 64 bits: fp32 accumulation in any order, K 2^-23 sum |a w| (with
 margin 2 over (K - 1) 2^-24), then one bf16 rounding (half an ulp of 8 significand bits: 2^-8 of the value); an
@@ -71,6 +71,49 @@ def test_gemm_bf16_strides_bias_and_edges(M, K, N):
         gemm_bf16(a, w, b, out=y[:M, :N])
         _check_bf16(y[:M, :N], a, w, b, False, None)
         assert bool((y[M:] == 3.0).all()) and bool((y[:, N:] == 3.0).all())
+
+
+def _bits(t):
+    return t.contiguous().view(torch.int16)
+
+
+@pytest.mark.parametrize("K,N,act,bias", [(1536, 1536, None, True), (1544, 9220, "silu", True), (4096, 1540, "gelu", False),
+                                          (72, 20, None, True), (8, 64, None, False), (520, 260, "gelu", True)])
+def test_gemm_bf16_rows_have_the_same_bits_in_any_call(K, N, act, bias):
+    """The first rows of calls of every size (few-row kernel at 8 and 16 rows and its 32-column workgroups, every
+    tile) against the direct kernel, which rows 8 MB apart reach (32-bit offsets end at 2 GiB)."""
+    a, w, b = _rand((2600, K), 21), _rand((N, K), 22, 0.05), _rand((N,), 23) if bias else None
+    apart = torch.zeros((20, 1 << 22), dtype=torch.bfloat16, device=DEV)
+    apart[:, :K] = a[:20]
+    ref = gemm_bf16(apart[:, :K], w, b, act_out=act)
+    _check_bf16(ref, a[:20], w, b, False, act)
+    for M in (1, 3, 8, 9, 16, 17, 20, 64, 300, 512, 1100, 2600):
+        got = gemm_bf16(a[:M], w, b, act_out=act)
+        assert torch.equal(_bits(got[:20]), _bits(ref[:M])), M
+
+
+@pytest.mark.parametrize("K,N", [(1536, 9216), (1544, 1540), (264, 8196), (72, 20), (5120, 256)])
+def test_gemm_bf16_silu_rows_have_the_same_bits_in_any_call(K, N):
+    """With SiLU on the input: the few-row kernel (8, 16 and 32 rows at a time) against the direct one at 65 rows."""
+    a, w, b = _rand((65, K), 24), _rand((N, K), 25, 0.05), _rand((N,), 26)
+    ref = gemm_bf16(a, w, b, silu_in=True)
+    _check_bf16(ref, a, w, b, True, None)
+    for M in (1, 7, 8, 9, 16, 17, 31, 32, 33, 64):
+        assert torch.equal(_bits(gemm_bf16(a[:M], w, b, silu_in=True)), _bits(ref[:M])), M
+
+
+def test_gemm_bf16_at_the_end_of_32_bit_offsets():
+    """The largest row stride that each form takes and the next one, which goes to the direct kernel: same bits."""
+    K, N = 264, 68
+    a, w, b = _rand((17, K), 27), _rand((N, K), 28, 0.05), _rand((N,), 29)
+    ref = gemm_bf16(a, w, b)
+    span = (1 << 31) - 16
+    for rows, most in ((17, 17 + 256), (3, 32)):
+        last = (span - 1) // (2 * most) // 8 * 8   # rows of the form's own count stay below the span
+        for lda in (last, last + 8):
+            x = torch.empty((rows * lda,), dtype=torch.bfloat16, device=DEV).as_strided((rows, K), (lda, 1))
+            x.copy_(a[:rows])
+            assert torch.equal(_bits(gemm_bf16(x, w, b)), _bits(ref[:rows])), (rows, lda)
 
 
 def test_gemm_bf16_zero_without_bias_keeps_its_sign():

@@ -44,135 +44,163 @@ struct Bf16GemmArgs {
   int64_t lda, ldy;
   int M, N, K;
   int act;      // 0 none, 1 SiLU, 2 GELU(tanh)
-  int m_tiles;  // groups of kSkinnyRows rows
+  int m_tiles;  // the few-row kernel's groups of rows
 };
 
 constexpr int kWaves = 4;
 constexpr int kTileM = 64, kTileN = 128;
 
-constexpr int kSkinnyRows = 16;   // rows of A per workgroup
-constexpr int kSkinnyCols = 16;   // columns of y (rows of W) per workgroup
-constexpr int kSkinnyWaves = 4;   // waves per workgroup, which split K
-constexpr int kSkinnyRing = 4;    // pieces of 64 K elements a wave has in flight
-constexpr int kPieceBytes = kSkinnyCols * 128;
+constexpr int kSkinnyWaves = 4;  // streaming waves of a workgroup; one more wave multiplies
 
-// y for up to 16 rows of A (8 with NA = 1) and 16 rows of W, the few-row products of the time embedding.  The
-// bound is the stream of W: K goes to the four waves in pieces of 64 elements (whole 128-byte lines of every W
-// row), which each wave brings into its own LDS ring by DMA, four pieces ahead, without a barrier.  A piece of A
-// is loaded, SiLU'd and handed over in LDS by the wave itself, 16 bytes per lane, so that the activation costs
-// what the rows hold and not a 16-row tile.  v_mfma_f32_16x16x32_bf16 takes 16 bytes of one row per lane (row
-// l % 16, K elements 8 (l / 16) .. + 7); chunk c of row r lies at 16 (c ^ ((r / 2) % 8)).  The waves' partial
-// sums are added in wave order.
-template <bool SILU_IN, int NA>
-__global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_bf16_skinny_kernel(Bf16GemmArgs p) {
-  constexpr int P = kSkinnyRing;
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[kSkinnyWaves * (P * kPieceBytes + kSkinnyRows * 128)];
+// y for 8 NA rows of A and 16 NB rows of W, the few-row products of the time embedding.  The bound is the stream
+// of W: K goes to the four streaming waves in pieces of 64 elements (whole 128-byte lines of every W row), which
+// each of them brings into its own LDS ring of P pieces by DMA.  A piece of A is loaded, SiLU'd and handed over in
+// LDS by the wave itself, 16 bytes per lane, so that the activation costs what the rows hold and not a 16-row tile.
+// After each step of four pieces a barrier hands them to the fifth wave, which alone multiplies, in K order: one
+// 16x16x32 MFMA adds in the order of the two 32x32x16 MFMAs of the other kernels, so a row has the same bits
+// whichever kernel its call takes.  v_mfma_f32_16x16x32_bf16 takes 16 bytes of one row per lane (row l % 16, K
+// elements 8 (l / 16) .. + 7); chunk c of row r lies at 16 (c ^ ((r / 2) % 8)).
+template <bool SILU_IN, int NA, int NB>
+__global__ __launch_bounds__((kSkinnyWaves + 1) * 64) void gemm_bf16_skinny_kernel(Bf16GemmArgs p) {
+  constexpr int P = NB == 1 ? 4 : 3, S = kSkinnyWaves;
+  constexpr int ROWS = 8 * NA, COLS = 16 * NB, MB = (NA + 1) / 2;
+  constexpr int APIECE = ROWS * 128, WPIECE = COLS * 128;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[S * P * WPIECE + 2 * S * APIECE];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r16 = lane & 15, kq = lane >> 4;
-  const int m0 = static_cast<int>(blockIdx.x % static_cast<uint32_t>(p.m_tiles)) * kSkinnyRows;
-  const int n0 = static_cast<int>(blockIdx.x / static_cast<uint32_t>(p.m_tiles)) * kSkinnyCols;
-  const int rows = min(p.M - m0, kSkinnyRows), cols = min(p.N - n0, kSkinnyCols);
-  uint8_t* const ring = lds + wave * (P * kPieceBytes);
-  uint8_t* const aw = lds + kSkinnyWaves * P * kPieceBytes + wave * (kSkinnyRows * 128);
-  // rows past M / N and chunks past K read zeros
-  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(p.a + static_cast<int64_t>(m0) * p.lda), 0,
-      ((rows - 1) * static_cast<int>(p.lda) + p.K) * 2, kBufferRsrcWord3);
-  const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(p.w + static_cast<int64_t>(n0) * p.K), 0, cols * p.K * 2, kBufferRsrcWord3);
-  // Lane l moves chunk l % 8 of row l / 8 (+ 8 i) of A, and of W the chunk that belongs at position l % 8 there.
-  const int r8 = lane >> 3, c8 = lane & 7;
-  u32x4 ar[P][NA];
-  int aoff[NA], woff[2], wk[2];
+  const int m0 = static_cast<int>(blockIdx.x % static_cast<uint32_t>(p.m_tiles)) * ROWS;
+  const int n0 = static_cast<int>(blockIdx.x / static_cast<uint32_t>(p.m_tiles)) * COLS;
+  const int steps = ((p.K + 63) / 64 + S - 1) / S;  // the last pieces may be past K: zeros
+  uint8_t* const abuf = lds + S * P * WPIECE;  // A's pieces of a step, two steps in turn
+
+  if (wave < S) {
+    const int rows = min(p.M - m0, ROWS), cols = min(p.N - n0, COLS);
+    uint8_t* const ring = lds + wave * (P * WPIECE);
+    // rows past M / N and chunks past K read zeros
+    const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(p.a + static_cast<int64_t>(m0) * p.lda), 0,
+        ((rows - 1) * static_cast<int>(p.lda) + p.K) * 2, kBufferRsrcWord3);
+    const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(p.w + static_cast<int64_t>(n0) * p.K), 0, cols * p.K * 2, kBufferRsrcWord3);
+    // Lane l moves chunk l % 8 of row l / 8 (+ 8 i) of A, and of W the chunk that belongs at position l % 8 there.
+    const int r8 = lane >> 3, c8 = lane & 7;
+    u32x4 ar[P][NA];
+    int aoff[NA], woff[2 * NB], wk[2 * NB];
 #pragma unroll
-  for (int i = 0; i < NA; ++i) aoff[i] = ((r8 + 8 * i) * static_cast<int>(p.lda) + 8 * c8) * 2;
+    for (int i = 0; i < NA; ++i) aoff[i] = ((r8 + 8 * i) * static_cast<int>(p.lda) + 8 * c8) * 2;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    wk[i] = 8 * (c8 ^ (((r8 + 8 * i) >> 1) & 7));
-    woff[i] = ((r8 + 8 * i) * p.K + wk[i]) * 2;
-  }
-  auto load = [&](auto S, int piece) {
-    constexpr int s = decltype(S)::value;
-    const int k0 = 64 * (wave + kSkinnyWaves * piece);
+    for (int i = 0; i < 2 * NB; ++i) {
+      wk[i] = 8 * (c8 ^ (((r8 + 8 * i) >> 1) & 7));
+      woff[i] = ((r8 + 8 * i) * p.K + wk[i]) * 2;
+    }
+    auto load = [&](auto SLOT, int step) {
+      constexpr int s = decltype(SLOT)::value;
+      const int k0 = 64 * (wave + S * step);
 #pragma unroll
-    for (int i = 0; i < NA; ++i)
-      ar[s][i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, k0 + 8 * c8 < p.K ? aoff[i] + 2 * k0 : kOutOfRange, 0, 0);
+      for (int i = 0; i < NA; ++i)
+        ar[s][i] =
+            __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, k0 + 8 * c8 < p.K ? aoff[i] + 2 * k0 : kOutOfRange, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-      dma16(rsrc_w, ring + s * kPieceBytes + i * 1024, k0 + wk[i] < p.K ? woff[i] + 2 * k0 : kOutOfRange);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  v4f acc = {0, 0, 0, 0};
-  const int x = (r16 >> 1) & 7;
-  auto compute = [&](auto S) {
-    constexpr int s = decltype(S)::value;
-    // this piece's loads landed; those of the P - 1 pieces behind it may be in flight
-    wait_counts<(P - 1) * (2 + NA), 15>();
-    asm volatile("" ::: "memory");
+      for (int i = 0; i < 2 * NB; ++i)
+        dma16(rsrc_w, ring + s * WPIECE + i * 1024, k0 + wk[i] < p.K ? woff[i] + 2 * k0 : kOutOfRange);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto hand_over = [&](auto SLOT, int step) {
+      constexpr int s = decltype(SLOT)::value;
+      uint8_t* const aw = abuf + (step & 1) * (S * APIECE) + wave * APIECE;
+      // this piece's loads landed; those of the P - 2 pieces behind it may be in flight
+      wait_counts<(P - 2) * (2 * NB + NA), 15>();
+      asm volatile("" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      u32x4 v = ar[s][i];
-      if constexpr (SILU_IN) {
+      for (int i = 0; i < NA; ++i) {
+        u32x4 v = ar[s][i];
+        if constexpr (SILU_IN) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = pack_bf16x2_hw(silu(bf16_lo_to_f32(v[e])), silu(bf16_hi_to_f32(v[e])));
+          for (int e = 0; e < 4; ++e) v[e] = pack_bf16x2_hw(silu(bf16_lo_to_f32(v[e])), silu(bf16_hi_to_f32(v[e])));
+        }
+        const int r = r8 + 8 * i;
+        *reinterpret_cast<u32x4*>(aw + r * 128 + 16 * (c8 ^ ((r >> 1) & 7))) = v;
       }
-      const int r = r8 + 8 * i;
-      *reinterpret_cast<u32x4*>(aw + r * 128 + 16 * (c8 ^ ((r >> 1) & 7))) = v;
+      wait_counts<63, 0>();
+      if (step <= steps) __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    };
+    static_for<P - 1>([&](auto I) { load(I, decltype(I)::value); });
+    // Whole rounds of the ring: with an exit inside, the compiler would wait at the top for loads that are to stay in
+    // flight.  Steps past the last hand over nothing; the first of them waits until the last is read.
+    for (int i = 0; i < steps; i += P) {
+      static_for<P>([&](auto I) {
+        constexpr int s = decltype(I)::value;
+        hand_over(I, i + s);
+        load(ic<(s + P - 1) % P>{}, i + s + P - 1);  // the slot of step i + s - 1, read before this step's barrier
+      });
     }
-    // read back by other lanes of this wave: LDS executes a wave's accesses in order (with NA = 1 rows 8.. hold
-    // whatever is there; they only reach rows of y that are not stored)
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    v8bf av[2], wv[2];
+    wait_counts<0, 0>();  // nothing of this wave is under way to LDS when it ends
+    return;
+  }
+
+  const int r16 = lane & 15, kq = lane >> 4;
+  auto at = [&](int r, int u) { return r * 128 + 16 * ((4 * u + kq) ^ ((r >> 1) & 7)); };
+  // the lane's rows m0 + 16 i + l % 16, columns n0 + 16 j + 4 (l / 16) .. + 3 (N % 4 == 0: all inside N or none)
+  const int m = m0 + r16, n = n0 + 4 * kq;
+  float bias[NB][4];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int at = r16 * 128 + 16 * ((4 * u + kq) ^ x);
-      wv[u] = *reinterpret_cast<const v8bf*>(ring + s * kPieceBytes + at);
-      av[u] = *reinterpret_cast<const v8bf*>(aw + at);
-    }
+  for (int j = 0; j < NB; ++j)
 #pragma unroll
-    for (int u = 0; u < 2; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[u], av[u], acc, 0, 0, 0);
-    // the piece's fragments are in registers before its slot is filled again
+    for (int e = 0; e < 4; ++e) bias[j][e] = -0.f;  // no bias: -0, which leaves every sum as it is
+  if (p.bias != nullptr) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bias[j][e] = bf16_bits_to_f32(p.bias[min(n + 16 * j, p.N - 4) + e]);
+  }
+  v4f acc[NB][MB] = {};
+  for (int i = 0; i < steps; ++i) {
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const uint8_t* const wp = lds + (i % P) * WPIECE;
+    const uint8_t* const ap = abuf + (i & 1) * (S * APIECE);
+    v8bf av[S][2][MB], wv[S][2][NB];
+#pragma unroll
+    for (int w = 0; w < S; ++w)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          wv[w][u][j] = *reinterpret_cast<const v8bf*>(wp + w * (P * WPIECE) + at(16 * j + r16, u));
+#pragma unroll
+        for (int b = 0; b < MB; ++b)  // (NA = 1: rows 8.. are rows 0.. again, and not stored)
+          av[w][u][b] = *reinterpret_cast<const v8bf*>(ap + w * APIECE + at((16 * b + r16) & (ROWS - 1), u));
+      }
+#pragma unroll
+    for (int w = 0; w < S; ++w)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int b = 0; b < MB; ++b)
+            acc[j][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[w][u][j], av[w][u][b], acc[j][b], 0, 0, 0);
+    // the step's fragments are in registers before the next barrier frees their slots
     wait_counts<63, 0>();
     asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  const int pieces = ((p.K + 63) / 64 + kSkinnyWaves - 1) / kSkinnyWaves;  // the last ones of a wave may be past K
-  static_for<P>([&](auto S) { load(S, decltype(S)::value); });
-  for (int i = 0; i < pieces; i += P) {
-    static_for<P>([&](auto S) {
-      constexpr int s = decltype(S)::value;
-      compute(S);                 // past the end: zeros
-      load(S, i + s + P);
-    });
   }
-  wait_counts<0, 0>();
-  __syncthreads();
-  v4f* const red = reinterpret_cast<v4f*>(lds);
-  red[wave * 64 + lane] = acc;
-  __syncthreads();
-  if (wave > 0) return;
-  // the lane's row m0 + l % 16, columns n0 + 4 (l / 16) .. + 3
-  v4f t = acc;
+  if (steps % P != 0) __builtin_amdgcn_s_barrier();  // of the first step past the last
 #pragma unroll
-  for (int s = 1; s < kSkinnyWaves; ++s) {
-    const v4f o = red[s * 64 + lane];
+  for (int j = 0; j < NB; ++j)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) t[e] = t[e] + o[e];
-  }
-  const int m = m0 + r16, n = n0 + 4 * kq;
-  if (m >= p.M || n >= p.N) return;
-  float v[4];
+    for (int b = 0; b < MB; ++b) {
+      if (m + 16 * b >= min(p.M, m0 + ROWS) || n + 16 * j >= p.N) continue;
+      float v[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    v[e] = bf16_round(p.bias ? __fadd_rn(t[e], bf16_bits_to_f32(p.bias[n + e])) : t[e]);
-    if (p.act == 1) v[e] = silu(v[e]);
-    if (p.act == 2) v[e] = gelu_tanh(v[e]);
-  }
-  *reinterpret_cast<uint2*>(p.y + static_cast<int64_t>(m) * p.ldy + n) =
-      make_uint2(pack_bf16x2_hw(v[0], v[1]), pack_bf16x2_hw(v[2], v[3]));
+      for (int e = 0; e < 4; ++e) {
+        v[e] = bf16_round(__fadd_rn(acc[j][b][e], bias[j][e]));
+        if (p.act == 1) v[e] = silu(v[e]);
+        if (p.act == 2) v[e] = gelu_tanh(v[e]);
+      }
+      *reinterpret_cast<uint2*>(p.y + static_cast<int64_t>(m + 16 * b) * p.ldy + n + 16 * j) =
+          make_uint2(pack_bf16x2_hw(v[0], v[1]), pack_bf16x2_hw(v[2], v[3]));
+    }
 }
 
 template <bool SILU_IN>
@@ -311,11 +339,16 @@ __global__ __launch_bounds__(256) void unpatchify_x0_kernel(const uint16_t* __re
   *reinterpret_cast<uint32_t*>(out + (((b * F + f) * C + c) * H + yy) * static_cast<int64_t>(W) + 2 * xp) = o;
 }
 
+template <bool SILU_IN, int NA, int NB>
+void launch_skinny(Bf16GemmArgs p, hipStream_t st) {
+  p.m_tiles = (p.M + 8 * NA - 1) / (8 * NA);
+  const int64_t blocks = static_cast<int64_t>(p.m_tiles) * ((p.N + 16 * NB - 1) / (16 * NB));
+  hipLaunchKernelGGL((gemm_bf16_skinny_kernel<SILU_IN, NA, NB>), dim3(static_cast<uint32_t>(blocks)),
+                     dim3((kSkinnyWaves + 1) * 64), 0, st, p);
+}
 template <bool SILU_IN, int NA>
-void launch_skinny(const Bf16GemmArgs& p, hipStream_t st) {
-  const int64_t blocks = static_cast<int64_t>(p.m_tiles) * ((p.N + kSkinnyCols - 1) / kSkinnyCols);
-  hipLaunchKernelGGL((gemm_bf16_skinny_kernel<SILU_IN, NA>), dim3(static_cast<uint32_t>(blocks)),
-                     dim3(kSkinnyWaves * 64), 0, st, p);
+void launch_skinny(bool wide, const Bf16GemmArgs& p, hipStream_t st) {
+  wide ? launch_skinny<SILU_IN, NA, 2>(p, st) : launch_skinny<SILU_IN, NA, 1>(p, st);
 }
 
 template <bool SILU_IN>
@@ -355,22 +388,26 @@ int wf_gemm_bf16(const void* a, int64_t m, int64_t k, int64_t lda, const void* w
   wf::Bf16GemmArgs p{static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(w),
                      static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(y), lda, ldy,
                      static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), act, 0};
-  // Few rows (the time embedding's 1-21 frames): the W stream's kernel; 3 x 1536 -> 9216 with SiLU 9.4 us against
-  // 40.7 us for the direct kernel (28.3 MB of W), 3 x 5120 -> 30720 57 us (5.5 TB/s).  It takes 16 rows at a time
-  // and W again for each 16, so without SiLU the tiles take over at 17 rows (21 x 1536 -> 1536: 5.9 against
-  // 7.8 us); with it, which only this kernel and the direct one apply, at 65.
-  const int64_t skinny_max = silu_in ? 64 : wf::kSkinnyRows;
-  if (m <= skinny_max && wf::product_below({wf::kSkinnyRows, lda, 2}, kSpan) &&
-      wf::product_below({wf::kSkinnyCols, k, 2}, kSpan)) {
-    p.m_tiles = static_cast<int>((m + wf::kSkinnyRows - 1) / wf::kSkinnyRows);
-    if (silu_in)
-      m <= 8 ? wf::launch_skinny<true, 1>(p, st) : wf::launch_skinny<true, 2>(p, st);
+  // Few rows (the time embedding's 1-21 frames): the W stream's kernel; 3 x 1536 -> 9216 with SiLU 6.6 us against
+  // 35.1 us for the direct kernel (28.3 MB of W), 3 x 5120 -> 30720 49.8 us (6.3 TB/s) against 148.  Without SiLU the
+  // tiles take over at 17 rows (17 x 1536 -> 1536: 4.8 us); with it, which only this kernel and the direct one apply,
+  // at 65.  Above 8 rows the SiLU that every workgroup repeats costs as much as the stream: where 32-column
+  // workgroups still give each CU one they halve it (16 x 5120 -> 30720: 58 against 69 us; 16 x 4096 -> 1536, which
+  // they would leave to 48 CUs, 9.5 against 6.4), and from 17 rows on take 32 rows at a time (21 x 1536 -> 9216:
+  // 13.6 against 18.0 us).
+  const int64_t skinny_max = silu_in ? 64 : 16;
+  if (m <= skinny_max && wf::product_below({32, lda, 2}, kSpan) && wf::product_below({32, k, 2}, kSpan)) {
+    const bool wide = (n + 31) / 32 >= wf::gemm::device_cus();
+    if (silu_in && wide && m > 16)
+      wf::launch_skinny<true, 4, 2>(p, st);
+    else if (silu_in)
+      m <= 8 ? wf::launch_skinny<true, 1, 1>(p, st) : wf::launch_skinny<true, 2>(wide, p, st);
     else
-      m <= 8 ? wf::launch_skinny<false, 1>(p, st) : wf::launch_skinny<false, 2>(p, st);
+      m <= 8 ? wf::launch_skinny<false, 1, 1>(p, st) : wf::launch_skinny<false, 2>(wide, p, st);
     return wf::check_launch(fn);
   }
-  // LDS-tiled: 512 x 4096 -> 1536 with GELU 15.0 us against 97.8 us, 4680 x 1536 -> 64 (head) 7.5 against 28.6 us,
-  // 4680 x 64 -> 1536 (patch embedding) 8.4 against 13.2 us for the direct kernel.
+  // LDS-tiled: 512 x 4096 -> 1536 with GELU 14.3 us against 97 us, 4680 x 1536 -> 64 (head) 5.0 against 28.5 us,
+  // 4680 x 64 -> 1536 (patch embedding) 8.1 against 13.3 us for the direct kernel.
   if (!silu_in && wf::product_below({m + 256, lda, 2}, kSpan) && wf::product_below({n + 256, k, 2}, kSpan)) {
     const wf::gemm::SmallArgs q{a, w, nullptr, nullptr, p.bias, p.y, p.M, p.N, 2 * p.K, static_cast<int>(2 * lda), ldy,
                                 ldy % 8 == 0 && wf::a16(y), (reinterpret_cast<uintptr_t>(bias) & 7u) == 0};

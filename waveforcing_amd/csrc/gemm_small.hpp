@@ -4,14 +4,17 @@
 // What bounds it: with few tiles neither the matrix cores nor memory, but the time of one K step in a workgroup
 // (barrier, fragment reads, a chain of MFMAs) times the steps, and below that the operand stream, (BM + BN) rows
 // of K through the 64 B/clk vector-memory path of one CU.  So the tiles are small (more CUs share the stream), the
-// smallest split K over groups of waves, fragments are read a step ahead of their MFMAs, and the LDS ring keeps up
-// to ST - 1 steps in flight.  Bytes move global -> LDS by DMA in the layout of gemm_w8a8.hip (1 KB blocks of 8 rows,
-// K chunks swizzled by the row), and without a K split every output sees the same MFMAs in the same K order as
-// there: bit-identical results (int32 sums with a split, too).
+// smallest keep two kinds of work side by side, fragments are read a step ahead of their MFMAs, and the LDS ring keeps
+// up to ST - 1 steps in flight.  Side by side: int8 splits K over groups of waves (int32 sums have the same bits in any
+// order); bf16, whose fp32 sums do not, gives the DMAs to waves of their own.  Bytes move global -> LDS by DMA in
+// the layout of gemm_w8a8.hip (1 KB blocks of 8 rows, K chunks swizzled by the row), and every fp32 sum takes the
+// same MFMAs in the same K order as there and in the other bf16 kernels: the bits of an output do not depend on
+// the tile, nor on the call's other rows.
 //
-// One K step: wait for the own DMAs of step kb, barrier (every wave's have landed and every wave is done with
+// One K step (DN = 0): wait for the own DMAs of step kb, barrier (every wave's have landed and every wave is done with
 // step kb - 1's stage), read step kb's fragments, DMA step kb + ST - 1 into that freed stage, then the MFMAs of
-// step kb - 1.  DMAs past K read zeros into stages that nobody reads any more.
+// step kb - 1.  DMAs past K read zeros into stages that nobody reads any more.  With DN loading waves these wait and
+// DMA, the others read and multiply, and the barrier of a step joins both.
 #pragma once
 
 #include <type_traits>
@@ -22,23 +25,25 @@ namespace wf {
 namespace gemm {
 
 // BM x BN outputs per workgroup of KS groups of WM x WN waves, each wave (BM / WM) x (BN / WN) in 32 x 32 blocks;
-// group g takes K steps g, g + KS, ... through its own ring of ST LDS stages, and the groups' sums are added at
-// the end (KS > 1 changes the order of fp32 sums, never an int32 one).
-template <int BM_, int BN_, int WM_, int WN_, int ST_, int KS_ = 1>
+// group g takes K steps g, g + KS, ... of U x 128 bytes through its own ring of ST LDS stages, and the groups' sums
+// are added at the end (int8 only: KS > 1 changes the order of sums).  DN > 0: DN more waves issue all DMAs.
+template <int BM_, int BN_, int WM_, int WN_, int ST_, int KS_ = 1, int U_ = 1, int DN_ = 0>
 struct SmallTile {
-  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, ST = ST_, KS = KS_;
-  static constexpr int NW = WM * WN, THREADS = KS * NW * 64;  // NW: waves of one group
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, ST = ST_, KS = KS_, U = U_, DN = DN_;
+  static constexpr int NW = WM * WN, THREADS = (KS * NW + DN) * 64;  // NW: waves of one group
+  static constexpr int NL = DN > 0 ? DN : NW;                        // waves that load
   static constexpr int MI = BM / WM / 32, NI = BN / WN / 32;
-  static constexpr int NBA = BM / 8 / NW, NBB = BN / 8 / NW, NDMA = NBA + NBB;
-  static constexpr int STAGE = (BM + BN) * BK;
+  static constexpr int NBA = BM / 8 / NL, NBB = BN / 8 / NL, NDMA = NBA + NBB;
+  static constexpr int CHUNK = (BM + BN) * BK, STAGE = U * CHUNK;
   static constexpr int WPITCH = BN / WN * 2 + 16;   // row pitch of a wave's 32-row output slab
   static constexpr int SLABS = MI > 1 ? 2 : 1;
   static_assert(MI >= 1 && NI >= 1 && MI * WM * 32 == BM && NI * WN * 32 == BN, "32 x 32 blocks");
-  static_assert(NBA * 8 * NW == BM && NBB * 8 * NW == BN, "DMA blocks");
-  static_assert(ST >= 3 && NDMA * (ST - 2) < 64, "outstanding DMAs");
+  static_assert(NBA * 8 * NL == BM && NBB * 8 * NL == BN, "DMA blocks");
+  static_assert(ST >= 3 && U * NDMA * (ST - 2) < 64, "outstanding DMAs");
   static constexpr int LDS = KS * ST * STAGE;
   static constexpr int ACC = MI * NI * 64 * 64;     // one wave's sums (bytes)
   static_assert(NW * SLABS * 32 * WPITCH <= LDS && LDS <= 160 * 1024, "LDS of one workgroup");
+  static_assert(DN == 0 || KS == 1, "loading waves of their own serve one group");
   static_assert(KS == 1 || (KS - 1) * NW * ACC <= LDS, "the groups' sums fit the stages");
 };
 
@@ -63,7 +68,7 @@ __global__ __launch_bounds__(T::THREADS) void gemm_small_kernel(SmallArgs p) {
   constexpr bool kI8 = std::is_same<OP, OpI8>::value, kFp8 = std::is_same<OP, OpFp8>::value;
   constexpr int SUB = OP::SUB, PIECES = OP::PIECES;
   constexpr int CPS = BK / 16 / SUB;
-  constexpr int KS = T::KS;
+  constexpr int KS = T::KS, U = T::U, DN = T::DN, NL = T::NL;
   __shared__ __attribute__((aligned(1024))) uint8_t lds_all[T::LDS];
 
   // Tiles in bands of GROUP_M tile rows swept column by column, a contiguous range of them per XCD.
@@ -81,6 +86,7 @@ __global__ __launch_bounds__(T::THREADS) void gemm_small_kernel(SmallArgs p) {
   const int lane = threadIdx.x & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wave = KS > 1 ? wave_all % NW : wave_all, ks = KS > 1 ? wave_all / NW : 0;
+  const int lwave = DN > 0 ? wave_all - NW : wave;  // of the loading waves
   uint8_t* const lds = lds_all + ks * (ST * STAGE);
   const int wm = wave / WN, wn = wave % WN;
   const int l32 = lane & 31, half = lane >> 5;
@@ -90,34 +96,53 @@ __global__ __launch_bounds__(T::THREADS) void gemm_small_kernel(SmallArgs p) {
   const __amdgpu_buffer_rsrc_t rsrc_w =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.w), 0, p.N * p.kb, kBufferRsrcWord3);
 
-  // DMA block j of this wave: rows (j * NW + wave) * 8 .. + 7 of A (j < NBA) or of W.
+  // DMA block j of this wave: rows (j * NL + lwave) * 8 .. + 7 of A (j < NBA) or of W.
   int doff[NDMA], dcol[NDMA];
 #pragma unroll
   for (int j = 0; j < NDMA; ++j) {
     const bool is_a = j < NBA;
-    const int r = ((is_a ? j : j - NBA) * NW + wave) * 8 + (lane >> 3);
+    const int r = ((is_a ? j : j - NBA) * NL + lwave) * 8 + (lane >> 3);
     const int c = (lane & 7) ^ ((r >> 1) & 7);
     dcol[j] = c * 16;
     doff[j] = is_a ? (m0 + r) * p.lda + c * 16 : (n0 + r) * p.kb + c * 16;
   }
   // The group's step kb (step KS kb + ks of the whole) into stage STG.
-  auto dma_step = [&](int kb, auto STG) {
-    constexpr int stage = decltype(STG)::value;
-    const int k0 = (KS * kb + ks) * BK;
+  auto dma_step = [&](int kb, int stage) {
+    const int k0 = (KS * kb + ks) * (U * BK);
     auto issue = [&](auto WHOLE) {
-      static_for<NDMA>([&](auto J) {
-        constexpr int j = decltype(J)::value;
-        uint8_t* const dst = lds + stage * STAGE + (j < NBA ? j * NW : BM / 8 + (j - NBA) * NW) * 1024 + wave * 1024;
-        const int off = decltype(WHOLE)::value || dcol[j] < p.kb - k0 ? doff[j] + k0 : kOutOfRange;
+      static_for<U * NDMA>([&](auto J) {
+        constexpr int u = decltype(J)::value / NDMA, j = decltype(J)::value % NDMA;
+        uint8_t* const dst = lds + stage * STAGE + u * T::CHUNK +
+                             (j < NBA ? j * NL : BM / 8 + (j - NBA) * NL) * 1024 + lwave * 1024;
+        const int k = k0 + u * BK;
+        const int off = decltype(WHOLE)::value || dcol[j] < p.kb - k ? doff[j] + k : kOutOfRange;
         dma16(j < NBA ? rsrc_a : rsrc_w, dst, off);
       });
     };
     // a whole step within K needs no check per chunk (rows past M and N are past the buffers' ends)
-    if (k0 + BK <= p.kb)
+    if (k0 + U * BK <= p.kb)
       issue(ic<1>{});
     else
       issue(ic<0>{});
   };
+
+  const int nk = ((p.kb + BK - 1) / BK + KS * U - 1) / (KS * U);  // steps per group (a last one past K adds zeros)
+  if constexpr (DN > 0) {
+    if (wave_all >= NW) {
+#pragma unroll
+      for (int s = 0; s < ST - 1; ++s) dma_step(s, s);
+      for (int kb = 0, stage = ST - 1; kb < nk; ++kb) {
+        wait_counts<U * NDMA * (ST - 2), 15>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        dma_step(kb + ST - 1, stage);
+        stage = stage + 1 == ST ? 0 : stage + 1;
+      }
+      wait_counts<0, 0>();
+      __builtin_amdgcn_s_barrier();
+      return;
+    }
+  }
 
   // Epilogue operands of the lane's outputs (block (j, i): row m = l32, columns 8 g + 4 half + 0..3 of block j),
   // loaded ahead of the operand stream.  N % 4 == 0: a group of 4 columns is inside N or not at all.
@@ -172,15 +197,14 @@ __global__ __launch_bounds__(T::THREADS) void gemm_small_kernel(SmallArgs p) {
 #pragma unroll
     for (int i = 0; i < MI; ++i) acc[j][i] = typename OP::acc_t{};
 
-  const int nk = ((p.kb + BK - 1) / BK + KS - 1) / KS;  // steps per group (a last one past K adds zeros)
-  static_for<ST - 1>([&](auto S) { dma_step(decltype(S)::value, S); });
+  if constexpr (DN == 0) static_for<ST - 1>([&](auto S) { dma_step(decltype(S)::value, decltype(S)::value); });
   // Fragments in two register sets: step kb's are read while the MFMAs of step kb - 1 run.  The stages and the
   // sets are compile-time (the loop is unrolled over both), so a step costs no address arithmetic but its DMAs'.
-  v4i fa[2][SUB][MI][PIECES], fw[2][SUB][NI][PIECES];
+  v4i fa[2][U * SUB][MI][PIECES], fw[2][U * SUB][NI][PIECES];
   auto mma = [&](auto B) {
     constexpr int b = decltype(B)::value;
 #pragma unroll
-    for (int s = 0; s < SUB; ++s)
+    for (int s = 0; s < U * SUB; ++s)
 #pragma unroll
       for (int j = 0; j < NI; ++j)
 #pragma unroll
@@ -190,23 +214,24 @@ __global__ __launch_bounds__(T::THREADS) void gemm_small_kernel(SmallArgs p) {
     constexpr int b = decltype(B)::value, stage = decltype(STG)::value;
     // own DMAs of step kb landed (those of the ST - 2 steps behind it may be in flight), own reads of the stage
     // before it done; the barrier makes both hold for every wave
-    wait_counts<NDMA * (ST - 2), 0>();
-    if constexpr (KS * NW > 1) __builtin_amdgcn_s_barrier();
+    wait_counts<DN == 0 ? U * NDMA * (ST - 2) : 63, 0>();
+    if constexpr (KS * NW + DN > 1) __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    const uint8_t* st = lds + stage * STAGE;
 #pragma unroll
-    for (int s = 0; s < SUB; ++s)
+    for (int s = 0; s < U * SUB; ++s) {
+      const uint8_t* st = lds + stage * STAGE + s / SUB * T::CHUNK;
 #pragma unroll
       for (int e = 0; e < PIECES; ++e) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
-          fa[b][s][i][e] = *reinterpret_cast<const v4i*>(st + i * 32 * BK + (lane_a + koff[s][e]));
+          fa[b][s][i][e] = *reinterpret_cast<const v4i*>(st + i * 32 * BK + (lane_a + koff[s % SUB][e]));
 #pragma unroll
         for (int j = 0; j < NI; ++j)
-          fw[b][s][j][e] = *reinterpret_cast<const v4i*>(st + j * 32 * BK + (lane_b + koff[s][e]));
+          fw[b][s][j][e] = *reinterpret_cast<const v4i*>(st + j * 32 * BK + (lane_b + koff[s % SUB][e]));
       }
+    }
     __builtin_amdgcn_sched_barrier(0);
-    dma_step(kb + ST - 1, ic<(stage + ST - 1) % ST>{});
+    if constexpr (DN == 0) dma_step(kb + ST - 1, (stage + ST - 1) % ST);
     __builtin_amdgcn_sched_barrier(0);
   };
   fetch(ic<0>{}, ic<0>{}, 0);
@@ -227,15 +252,14 @@ __global__ __launch_bounds__(T::THREADS) void gemm_small_kernel(SmallArgs p) {
     mma(ic<1>{});
   // every DMA landed and every wave past its last LDS read before the stages are reused for the output staging
   wait_counts<0, 0>();
-  if constexpr (KS * NW > 1) __builtin_amdgcn_s_barrier();
+  if constexpr (KS * NW + DN > 1) __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 
   if constexpr (KS > 1) {
     // groups 1.. hand their sums to group 0 (16 bytes per lane and store), which adds them in group order and
     // finishes alone
-    typedef typename std::conditional<kI8, int, float>::type elem;
-    typedef elem v4e __attribute__((ext_vector_type(4)));
-    v4e* const sums = reinterpret_cast<v4e*>(lds_all);
+    static_assert(kI8, "only int32 sums may be split");
+    v4i* const sums = reinterpret_cast<v4i*>(lds_all);
     auto at = [&](int g, int j, int i, int q) { return (((((g - 1) * NW + wave) * NI + j) * MI + i) * 4 + q) * 64 + lane; };
     if (ks > 0) {
 #pragma unroll
@@ -245,7 +269,7 @@ __global__ __launch_bounds__(T::THREADS) void gemm_small_kernel(SmallArgs p) {
 #pragma unroll
           for (int q = 0; q < 4; ++q)
             sums[at(ks, j, i, q)] =
-                v4e{acc[j][i][4 * q], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]};
+                v4i{acc[j][i][4 * q], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]};
     }
     __syncthreads();
     if (ks == 0) {
@@ -257,7 +281,7 @@ __global__ __launch_bounds__(T::THREADS) void gemm_small_kernel(SmallArgs p) {
           for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-              const v4e o = sums[at(g, j, i, q)];
+              const v4i o = sums[at(g, j, i, q)];
 #pragma unroll
               for (int e = 0; e < 4; ++e) acc[j][i][4 * q + e] += o[e];
             }
@@ -330,14 +354,19 @@ void launch_small(const SmallArgs& p, hipStream_t stream) {
   hipLaunchKernelGGL((gemm_small_kernel<T, OP, ACT>), grid, dim3(T::THREADS), 0, stream, p);
 }
 
-// The tiles.  In-workgroup split of K (KS) for the two small ones, whose time is the latency of a K step (about
-// 350-450 cycles whatever its bytes); e4m3 keeps one group, so that its fp32 sums keep the order they have in the
-// large tiles.
+// The tiles.  The time of the two small ones is the latency of a K step (about 350-450 cycles whatever its bytes).
+// int8 runs groups of waves beside each other (KS).  bf16 has waves that only load, and two 128-byte chunks per step:
+// 64 x 1536 -> 1536 4.9 us, 512 x 4096 -> 1536 14.3 us; the waves loading for themselves 6.3 and 16.8, a K split
+// (another order of the sums) 5.7 and 14.8.  e4m3 keeps one group that loads for itself.
 template <typename OP>
 struct SmallTiles {
-  static constexpr bool split = !std::is_same<OP, OpFp8>::value;
-  using T0 = typename std::conditional<split, SmallTile<32, 64, 1, 2, 3, 4>, SmallTile<32, 64, 1, 2, 6>>::type;
-  using T1 = typename std::conditional<split, SmallTile<64, 64, 2, 2, 4, 2>, SmallTile<64, 64, 2, 2, 4>>::type;
+  static constexpr bool i8 = std::is_same<OP, OpI8>::value, bf16 = std::is_same<OP, OpBf16>::value;
+  using T0 = typename std::conditional<
+      i8, SmallTile<32, 64, 1, 2, 3, 4>,
+      typename std::conditional<bf16, SmallTile<32, 64, 1, 2, 4, 1, 2, 4>, SmallTile<32, 64, 1, 2, 6>>::type>::type;
+  using T1 = typename std::conditional<
+      i8, SmallTile<64, 64, 2, 2, 4, 2>,
+      typename std::conditional<bf16, SmallTile<64, 64, 2, 2, 4, 1, 2, 4>, SmallTile<64, 64, 2, 2, 4>>::type>::type;
   using T2 = SmallTile<64, 128, 2, 4, 3>;
   using T3 = SmallTile<128, 128, 2, 4, 4>;
 };

@@ -65,6 +65,7 @@
 // it) moves P by percents.
 #include <utility>
 
+#include "attn_split.hpp"
 #include "fastdiv.hpp"
 #include "fp8_codec.hpp"
 #include "gemm_core.hpp"
@@ -840,35 +841,10 @@ __global__ __launch_bounds__(THREADS, 1) void attn_paged_fp8_kernel(AttnArgs p) 
 
 }  // namespace
 
-// Queries per workgroup: the split whose rounds of workgroups (one per CU) take least.  Cost of a round against
-// the 128-query split's, measured per tile over the four forms: 256 queries 1.55-1.67, 96 queries 0.92-1.0, 64 and
-// 32 queries 0.90-0.97 (fewer query waves contend for LDS).  4680 queries x 12 heads: 228 workgroups of 256 in one
-// round (22.9 us over 512 keys) against 444 of 128 in two (27.7 us); 1560 x 40 heads x 10920 keys: 280 of 256 in
-// two rounds 577 us, 520 of 128 in three 491 us, 680 of 96 in three 476 us.
-int pick_queries(int64_t lq, int n_heads, int64_t n_kv) {
-  // the staging waves index up to four tiles past the last
-  if (n_kv >= (1ll << 31) - 8 * BKV) return BQ;
-  static constexpr struct {
-    int bq;
-    double cost;
-  } kSplits[] = {{BQ, 1.6}, {128, 1.0}, {96, 0.95}, {64, 0.94}, {32, 0.92}};
-  const int64_t cus = gemm::device_cus();
-  int best = BQ;
-  double best_cost = 0;
-  for (const auto& sp : kSplits) {
-    const int64_t items = (lq + sp.bq - 1) / sp.bq * n_heads;
-    const double cost = sp.cost * static_cast<double>((items + cus - 1) / cus);
-    if (sp.bq == BQ || cost < best_cost) {
-      best = sp.bq;
-      best_cost = cost;
-    }
-  }
-  return best;
-}
-
 template <bool DENSE, bool QK8, bool PV8>
 int launch_attn(AttnArgs p, int64_t lq, int n_heads, hipStream_t stream) {
-  p.bq = pick_queries(lq, n_heads, p.n_kv);
+  static_assert(BQ == kQueriesWide && BKV == kTileKeys, "the split's rule counts these");
+  p.bq = pick_queries(lq, n_heads, p.n_kv, QK8, gemm::device_cus());
   const int64_t items = (lq + p.bq - 1) / p.bq * n_heads;
   const dim3 grid(static_cast<uint32_t>((items + 7) / 8 * 8));
   if (p.bq == BQ)

@@ -13,7 +13,8 @@ import torch
 
 from waveforcing_amd import _lib, inputs
 from waveforcing_amd.backend import attn_dense_bf16, attn_paged_fp8
-from waveforcing_amd.fp8 import gemm_i8
+from waveforcing_amd.dit import gemm_bf16
+from waveforcing_amd.fp8 import gemm_fp8_pertensor, gemm_i8
 from waveforcing_amd.kv import Fp8PagePool, PagedKV
 
 pytestmark = pytest.mark.gpu
@@ -77,6 +78,34 @@ def test_gemm_i8_repeats(M, N, K):
     y = torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
     acc = torch.empty((M, N), dtype=torch.int32, device=DEV)
     _assert_repeats(lambda: gemm_i8(qx, qw, sx, sw, bias, acc_out=acc, out=y), [y, acc])
+
+
+@pytest.mark.parametrize("M", [20, 64, 150, 300])
+def test_small_tile_gemms_repeat(M):
+    """The small GEMM tiles (32 x 64, 64 x 64, 64 x 128, 128 x 128 by M): int8, whose groups of waves add their sums
+    in LDS, e4m3, and bf16, whose first two have loading waves of their own."""
+    N, K = 8960, 1552
+    g = torch.Generator().manual_seed(M)
+    qx = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8).to(DEV)
+    qw = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8).to(DEV)
+    sx, sw = torch.rand(M, generator=g).to(DEV), torch.rand(N, generator=g).to(DEV)
+    a, w, bias = _normal((M, K), 14), _normal((N, K), 15), _normal((N,), 16)
+    a8, w8 = a.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+    s1 = torch.ones((1,), device=DEV)
+    y = torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
+    _assert_repeats(lambda: gemm_i8(qx, qw, sx, sw, bias, out=y), [y])
+    _assert_repeats(lambda: gemm_fp8_pertensor(a8, w8, s1, s1, bias, out=y), [y])
+    _assert_repeats(lambda: gemm_bf16(a, w, bias, out=y), [y])
+
+
+@pytest.mark.parametrize("M,N", [(3, 9216), (16, 1536), (16, 9216), (32, 9216)])
+@pytest.mark.parametrize("silu", [False, True])
+def test_few_row_gemm_repeats(M, N, silu):
+    """The few-row bf16 kernel at 8, 16 and (with SiLU) 32 rows per workgroup, 16 and 32 columns; 49 pieces of K, so
+    that the last step is partly past K."""
+    a, w, bias = _normal((M, 3104), 17), _normal((N, 3104), 18), _normal((N,), 19)
+    y = torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
+    _assert_repeats(lambda: gemm_bf16(a, w, bias, out=y, silu_in=silu), [y])
 
 
 def test_act_quant_repeats():

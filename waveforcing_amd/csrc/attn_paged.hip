@@ -39,7 +39,7 @@
 //   * the 32 V^T reads are issued before the softmax, so they land during it;
 //   * each 16-key step's exponentials feed its 4 PV MFMAs, so the
 //     exponentials of step t+1 issue under the MFMAs of step t.
-// A wave issues a VALU instruction at most every ~8 cycles on gfx950, so
+// A wave issues a VALU instruction every 5-6.5 cycles at most on gfx950, so
 // the vector work only hides when it sits between the wave's own MFMAs.
 //
 // Few queries (FEW): a grid of 256-query workgroups that leaves CUs idle is split finer instead.  Four waves own
@@ -47,9 +47,9 @@
 // light mate and issues nothing but its scores, softmax and PV: a tile takes 0.9-1.1 us instead of 1.5-1.8 us,
 // for at most half the queries.  The staging waves keep two further tiles in flight in registers.  Every query's
 // arithmetic is that of the 256-query form, so its output bits do not depend on the split.  1560 queries x 12
-// heads x 10920 keys, 84 -> 204 workgroups: exact 270 -> 157 us, quantized QK 310 -> 183, fp8 PV 306 -> 194; 300
-// queries x 5000 keys 128 -> 72, 147 -> 81, 145 -> 86; 48 queries x 3000 keys 77 -> 44, 80 -> 50, 83 -> 53;
-// dense 1560 x 10920 256 -> 154.  What bounds it now is one wave's issue rate (a VALU every 5-6.5 cycles, ~210
+// heads x 10920 N(0, 1) keys, 84 -> 204 workgroups: exact 274 -> 167 us, quantized QK 262 -> 155, fp8 PV 257 -> 164,
+// dense 261 -> 164; 300 queries x 5000 heavy-tailed keys 127 -> 72, 145 -> 81, 146 -> 86, 121 -> 73; 48 queries x 3000
+// 76 -> 44, 79 -> 50, 82 -> 53, 72 -> 45.  What bounds it now is one wave's issue rate (a VALU every 5-6.5 cycles, ~210
 // instructions per tile); running the next tile's score MFMAs under the softmax there gained 7 % (dense,
 // quantized QK) and lost 6 % (exact), so one body serves both splits.
 //

@@ -373,11 +373,15 @@ struct SmallTiles {
 
 // The tile of an M x N output with kb bytes of K, or -1 when `always` is false and the large tiles are the better
 // ones: the smallest tile that covers the output in one round of workgroups (one per CU), because a round's time
-// grows with the tile (int8, K = 1536 / 8960, us: 32 x 64 5.2 / 12.6, 64 x 64 5.7 / 15.4, 64 x 128 6.7 / 22.5,
-// 128 x 128 8.9 / 30.4, 128 x 256 11.5 / 40) and a second round costs more than the next tile up (512 x 1536 x 1536:
-// 32 x 64 in two rounds 9.2, 64 x 64 in one 6.0).  Past one round of 128 x 128 the 128 x 256 tile is ahead
-// (1560 x 4608 x 1536: 17.5 against 20.4).  A K of at most four steps is all launch, fill and stores: 64 x 128,
-// two workgroups per CU (4680 x 1536, K = 64 bf16: 8.4 against 10.5 / 39 us for 64 x 64 / 32 x 64).
+// grows with the tile and a second round costs more than the next tile up.  us of 32 x 64, 64 x 64, 64 x 128, 128 x 128
+// and 128 x 256 (M x N, K; where a rounds count is given, of more than one):
+//   int8  300 x 1536, 1536: 5.2 5.5 6.0 8.5 10.6     300 x 1536, 8960: 13.7 14.9 22.4 30.5 40.1
+//   e4m3  300 x 1536, 1536: 5.1 5.2 5.5 8.0 10.1     300 x 1536, 8960: 14.8 16.7 22.0 29.5 38.4
+//   bf16  300 x 1536, 1536: 5.5 5.9 8.3 12.5         300 x 5120, 4096: 39 (3 rounds) 26.5 (2) 23.4 31.2
+//   512 x 1536, 1536: int8 8.8 (2) 5.6 6.1, e4m3 5.9 (2) 5.3 5.6, bf16 9.4 (2) 6.2 8.4
+// Past one round of 128 x 128 the 128 x 256 tile is ahead (1560 x 4608, K = 1536: int8 16.8 against 19.6, e4m3 16.0
+// against 18.5).  A K of at most four steps is all launch, fill and stores: 64 x 128, two workgroups per CU
+// (4680 x 1536, K = 64 bf16: 8.1 against 17 / 25 us for 64 x 64 / 32 x 64).
 inline int pick_small(int M, int N, int kb, bool always) {
   if (g_tile_policy >= 2) return g_tile_policy - 2;
   const int64_t cus = device_cus();
